@@ -60,6 +60,9 @@ __host__ __device__ __forceinline__ Recip make_recip(double b) {
     return R;
 }
 struct DivFast {
+    __host__ __device__ __forceinline__ Recip recip(double b) { return make_recip(b); }
+    __host__ __device__ __forceinline__ void see(double) {}
+    __host__ __device__ __forceinline__ void in(bool) {}
     __host__ __device__ __forceinline__ double operator()(double a, const Recip &R) {
         const double q0 = a * R.r;
         const double rem = __builtin_fma(-R.b, q0, a);
@@ -74,6 +77,105 @@ struct DivFast {
 struct DivExact {
     __device__ __forceinline__ double operator()(double a, const Recip &R) { return a / R.b; }
 };
+
+// Quotients of operands known to be far from overflow and underflow: the
+// hardware reciprocal refined by two Newton steps, the quotient and one
+// residual correction.  These are the operations the division operator
+// expands to on this target, less its scaling and fix-up instructions, which
+// leave such operands and results alone: the same bits in 8 instructions
+// instead of 11, and without the mask register every scaled division passes
+// its flag through, so independent divisions overlap.  Sufficient: |a| and
+// |b| in [2^-300, 2^300], or a zero.  The residual is taken as b q0 - a so
+// that a zero a keeps its sign for b > 0.  near_rcp(b) serves several
+// numerators of one divisor.
+__device__ __forceinline__ double near_rcp(double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+    return __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+}
+__device__ __forceinline__ double div_mid(double a, double b, double r) {
+    const double q0 = a * r;
+    const double rem = __builtin_fma(b, q0, -a);
+    return __builtin_fma(-rem, r, q0);
+}
+__device__ __forceinline__ double div_mid(double a, double b) { return div_mid(a, b, near_rcp(b)); }
+
+// The high word of |x| less that of 2^LO as an unsigned number lies below this
+// span exactly when 2^LO <= |x| < 2^HI; NaN, infinities, zeros and, for the
+// signed form, negative x fall outside.
+template <int LO, int HI>
+__device__ __forceinline__ bool in_range(double x) {
+    return (uint32_t)__double2hiint(x) - (uint32_t)((1023 + LO) << 20) < (uint32_t)((HI - LO) << 20);
+}
+template <int LO, int HI>
+__device__ __forceinline__ bool abs_in_range(double x) {
+    return ((uint32_t)__double2hiint(x) << 1) - ((uint32_t)(1023 + LO) << 21) < ((uint32_t)(HI - LO) << 21);
+}
+
+// sqrtf of a float x that is zero or >= 2^-96 (NaN and infinity keep their
+// value), correctly rounded: the hardware root is within one unit in the last
+// place, so the result is it or a neighbour, and s s' >= x (or < x) tells on
+// which side of the midpoint of two neighbours s, s' the root lies (x and s s'
+// are multiples of the same power of two below which the midpoint's square
+// differs from s s').
+__device__ __forceinline__ float sqrt_mid(float x) {
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float lo = __uint_as_float(__float_as_uint(s) - 1u), hi = __uint_as_float(__float_as_uint(s) + 1u);
+    float r = __builtin_fmaf(-lo, s, x) <= 0.0f ? lo : s;
+    r = __builtin_fmaf(-hi, s, x) > 0.0f ? hi : r;
+    return r;
+}
+
+// Division policy of the FP64 stage: every quotient by the reciprocal form,
+// unchecked, with what the check needs accumulated beside it.  The caller
+// asks fails() once at the end and, if some lane's operands left the range,
+// evaluates the whole expression again with DivFast.  What has to hold is
+// DivFast's condition: every divisor in [2^-16, 2^100], every quotient zero or
+// in [2^-950, ...) (then the residual is a multiple of 2^-1074 and exactly
+// representable), nothing overflowed; a quotient that overflows or is NaN
+// makes the results NaN or infinite, which see() notes.  Quotients below
+// 2^-1042 count as zero.  DivFast compares, selects and branches at each of
+// about 300 divisions a cell and stage (three 64-bit compares, a select and a
+// branch each); here a division costs its four instructions and one and a
+// half 32-bit ones.  With nr_step_try the 3+1D kernel issues 2.36e8 VALU
+// instructions per launch at 131x131x61 where it issued 3.35e8; with their
+// copies, 60 steps of that event took 112.8 instead of 122.8 ms, 100 steps of
+// a 147x129 event 6.48 instead of 8.32 ms, 200 conformal steps at 201x201 9.87
+// instead of 12.2 ms, 40 steps of 16 batched events 16.6 instead of 18.9 ms.
+struct DivTry {
+    uint32_t lo = 0xffffffffu, hi = 0;
+    bool ok = true;
+    __device__ __forceinline__ Recip recip(double b) {
+        double r = near_rcp(b);
+        r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);  // 1/b correctly rounded
+        ok = ok && in_range<-16, 100>(b);
+        return Recip{b, r, true};
+    }
+    __device__ __forceinline__ double operator()(double a, const Recip &R) {
+        const double q0 = a * R.r;
+        const double rem = __builtin_fma(R.b, q0, -a);
+        const uint32_t u = ((uint32_t)__double2hiint(q0) << 1) + 0xffffffffu;  // zero becomes the largest
+        lo = u < lo ? u : lo;
+        return __builtin_fma(-rem, R.r, q0);
+    }
+    __device__ __forceinline__ void see(double x) {
+        const uint32_t u = (uint32_t)__double2hiint(x) << 1;
+        hi = u > hi ? u : hi;
+    }
+    __device__ __forceinline__ void in(bool inside) { ok = ok && inside; }
+    __device__ __forceinline__ bool fails() const {
+        return !ok || lo < ((1023u - 950u) << 21) - 1u || hi >= 0x7ffu << 21;
+    }
+};
+// The table lookups of DivTry's callers: their quotients need no check (a
+// quotient too small for the residual to be exact changes neither the index
+// nor the interpolated value, a NaN or infinite energy density gives the
+// same 1e-15 floor).
+struct DivTable {
+    __device__ __forceinline__ double operator()(double a, const Recip &R) { return div_mid(a, R.b, R.r); }
+};
+template <class DV>
+using TableDiv = std::conditional_t<std::is_same_v<DV, DivTry>, DivTable, DV>;
 
 // Quotient policies of the root solve and the primitive recovery.  QuotExact
 // is the division operator (the FP64 path).  QuotFast (mixed form only) is a
@@ -156,10 +258,11 @@ template <class DV>
 __device__ __forceinline__ double eos_interp(const EosDev &E, double e, const double *__restrict__ tb, DV &div) {
     const double e0 = E.e_min, de = E.e_spacing;
     const Recip Rde{de, E.r_spacing, true};
-    int idx = (int)div(e - e0, Rde);
+    TableDiv<DV> dt;
+    int idx = (int)dt(e - e0, Rde);
     idx = idx < EOS_LEN - 2 ? idx : EOS_LEN - 2;
     idx = idx > 0 ? idx : 0;
-    const double frac = div(e - (idx * de + e0), Rde);
+    const double frac = dt(e - (idx * de + e0), Rde);
     double t1 = tb[idx], t2 = tb[idx + 1];
     return t1 * (1. - frac) + t2 * frac;
 }
@@ -170,7 +273,8 @@ __device__ __forceinline__ double eos_pressure(const EosDev &E, double e, DV &di
         double f = eos_interp(E, e, E.p_tb, div);
         return 1.e-15 < f ? f : 1.e-15;  // std::max(1.e-15, f)
     } else {
-        return div(e, Recip{3., 1. / 3., true});
+        TableDiv<DV> dt;
+        return dt(e, Recip{3., 1. / 3., true});
     }
 }
 
@@ -197,7 +301,13 @@ __device__ __forceinline__ double eos_cs2(const EosDev &E, double e, DV &div) {
         double p = eos_pressure<true>(E, e, div);
         double p_r = eos_pressure<true>(E, e + delta_e, div);
         double delta_p = p_r - p;
-        double v = E.cs2_mode ? delta_p / delta_e : delta_e / delta_p;
+        double v;
+        if (E.cs2_mode) {
+            if constexpr (std::is_same_v<DV, DivTry>) v = div_mid(delta_p, delta_e, E.r_spacing);
+            else v = delta_p / delta_e;
+        } else {
+            v = delta_e / delta_p;
+        }
         v = v_max < v ? v_max : v;  // std::min(v_max, v)
         v = v_min < v ? v : v_min;  // std::max(v_min, .)
         return v;
@@ -234,6 +344,29 @@ __device__ __forceinline__ double approx_deriv(double x, double y, double z) {
     const double lo = __builtin_fmin(l, __builtin_fmin(c, r));
     const double hi = __builtin_fmax(l, __builtin_fmax(c, r));
     return __builtin_fmax(lo, __builtin_fmin(hi, 0.0)) + 0.0;
+}
+
+struct Prim {
+    double e, p, ut, ux, uy, un;
+};
+
+// getInferredVariables, rhic/src/EnergyMomentumTensor.cpp:117-233, in two
+// parts: the energy density from the conserved variables (the closed form
+// below ePrev = 0.1, else the root solve), then pressure, floors and
+// velocity.  ttt..pitn are q[0..7]; Pi = q[14] when bulk is evolved.
+struct Moments {
+    double M0, M1, M2, M3, M;
+};
+
+__device__ __forceinline__ Moments moments(double t, double ttt, double ttx, double tty, double ttn, double pitt,
+                                           double pitx, double pity, double pitn) {
+    Moments m;
+    m.M0 = ttt - pitt;
+    m.M1 = ttx - pitx;
+    m.M2 = tty - pity;
+    m.M3 = ttn - pitn;
+    m.M = m.M1 * m.M1 + m.M2 * m.M2 + t * t * m.M3 * m.M3;
+    return m;
 }
 
 // Newton-Raphson + bisection root solve of the table EoS,
@@ -284,6 +417,30 @@ __device__ __forceinline__ double nr_step(const EosDev &E, double e0, double M0,
     const double step = QD::q(f, fp);
     bad = __builtin_isnan(step);
     return e0 - step;
+}
+
+// nr_step's QuotExact form with the same bits from div_mid and sqrt_mid, and
+// ok cleared where an operand leaves their range: e0 in [2^-100, 2^100], H in
+// [2^-47, 2^60] and |f'| in [2^-60, 2^100] bound the others (p is 1e-15 or
+// more, |A| < 2^90 where H is bounded, A - H is zero or at least 2^-124; an
+// intermediate that overflows makes f' NaN, and one that underflows is too
+// small to change f').  e0's reciprocal serves both quotients by e0.  The
+// iteration is about half the instructions of the operator's, which spends
+// eleven on each of ten divisions and some twenty on the double square root.
+__device__ __forceinline__ double nr_step_try(const EosDev &E, double e0, double M0, double B, double Pi, DivTry &dx,
+                                              bool &ok) {
+    const double p = eos_pressure<true>(E, e0, dx);
+    const double cs2 = eos_cs2<true>(E, e0, dx);
+    const double r0 = near_rcp(e0);
+    const double cst2 = div_mid(p, e0, r0);
+    const double A = M0 * (1.0 - cst2) + Pi;
+    const double H = (double)sqrt_mid(f32_fabs((float)(A * A + 4 * cst2 * B)));
+    const double D = div_mid(A - H, 2 * cst2);
+    const double f = e0 + D;
+    const double fp = 1.0 - div_mid((cs2 - cst2) * (B + D * H - div_mid((cs2 - cst2) * cst2 * D * M0, e0, r0)),
+                                    cst2 * e0 * H);
+    ok = in_range<-100, 100>(e0) && in_range<-47, 60>(H) && abs_in_range<-60, 100>(fp);
+    return e0 - div_mid(f, fp);
 }
 
 // the reference's stop test, evaluated in float (:44); the mixed form
@@ -345,6 +502,43 @@ __device__ __forceinline__ RootResult table_root(const EosDev &E, double ePrev, 
         e0 = e;
     }
     return RootResult{table_bisect<QD, DV>(E, ePrev, M0, M, Pi), NAN_NONE};
+}
+
+// Table-EoS root solves from one start value, stepped together: table_root of
+// each state with nr_step_try.  Each takes exactly the steps table_root takes;
+// the N independent chains overlap.  A state that leaves nr_step_try's range
+// (a NaN among the causes), or has not converged after TRY_ITERS steps, ends
+// the attempt (ok false): the caller solves again with table_root, which
+// alone goes on to MAX_ITERS_NR and the bisection.
+constexpr int TRY_ITERS = 64;
+template <int N>
+__device__ __forceinline__ void table_roots_try(const EosDev &E, double ePrev, const Moments (&m)[N],
+                                                const double (&Pi)[N], double (&e)[N], bool &ok) {
+    DivTry dx;
+    double B[N];
+    bool done[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        B[k] = m[k].M0 * (m[k].M0 + Pi[k]) - m[k].M;
+        e[k] = ePrev;
+        done[k] = false;
+    }
+    bool any = true;
+    for (int j = 0; j < TRY_ITERS && any; ++j) {
+        any = false;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            if (!done[k]) {
+                bool in;
+                const double en = nr_step_try(E, e[k], m[k].M0, B[k], Pi[k], dx, in);
+                done[k] = nr_converged<QuotExact>(en, e[k]);
+                e[k] = en;
+                if (!in) ok = false;
+                any = any || !(done[k] || !in);
+            }
+        }
+    }
+    ok = ok && !any;
 }
 
 // The segment of E.p4 holding e (clamped to the table's ends, where its
@@ -429,36 +623,13 @@ __device__ __forceinline__ double energy_from_conserved(const EosDev &E, double 
     }
 }
 
-struct Prim {
-    double e, p, ut, ux, uy, un;
-};
-
-// getInferredVariables, rhic/src/EnergyMomentumTensor.cpp:117-233, in two
-// parts: the energy density from the conserved variables (the closed form
-// below ePrev = 0.1, else the root solve), then pressure, floors and
-// velocity.  ttt..pitn are q[0..7]; Pi = q[14] when bulk is evolved.
-struct Moments {
-    double M0, M1, M2, M3, M;
-};
-
-__device__ __forceinline__ Moments moments(double t, double ttt, double ttx, double tty, double ttn, double pitt,
-                                           double pitx, double pity, double pitn) {
-    Moments m;
-    m.M0 = ttt - pitt;
-    m.M1 = ttx - pitx;
-    m.M2 = tty - pity;
-    m.M3 = ttn - pitn;
-    m.M = m.M1 * m.M1 + m.M2 * m.M2 + t * t * m.M3 * m.M3;
-    return m;
-}
-
 template <bool TABLE, class DV, class QD>
 __device__ __forceinline__ Prim recover_finish(const EosDev &E, const Moments &m, double e, double Pi, int &nan,
                                                DV &div) {
     Prim r;
     r.e = e;
     if (__builtin_isnan(r.e)) nan = NAN_ENERGY;
-    constexpr bool FAST = std::is_same_v<QD, QuotFast>;
+    constexpr bool FAST = std::is_same_v<QD, QuotFast>, TRY = std::is_same_v<DV, DivTry>;
     if constexpr (FAST && TABLE) r.p = eos_pressure_fast(E, r.e);
     else r.p = eos_pressure<TABLE>(E, r.e, div);
     if (r.e < 1.e-7) {
@@ -466,13 +637,20 @@ __device__ __forceinline__ Prim recover_finish(const EosDev &E, const Moments &m
         r.p = 1.e-7;
     }
     double P = r.p + Pi;
-    double Ei;
-    if constexpr (FAST) Ei = QuotFast::rcp1(r.e + P);
-    else Ei = QD::q(1.0, r.e + P);
-    r.ut = (double)QD::sqrt_island(f32_fabs((float)((m.M0 + P) * Ei)));
-    double E2;
-    if constexpr (FAST) E2 = Ei * QuotFast::rcp1(r.ut);
-    else E2 = QD::q(Ei, r.ut);
+    double Ei, E2;
+    if constexpr (TRY) {
+        const double w = r.e + P;
+        Ei = div_mid(1.0, w);
+        r.ut = (double)sqrt_mid(f32_fabs((float)((m.M0 + P) * Ei)));
+        E2 = div_mid(Ei, r.ut);
+        div.ok = div.ok && in_range<-100, 100>(w) && in_range<-16, 100>(r.ut);
+    } else {
+        if constexpr (FAST) Ei = QuotFast::rcp1(r.e + P);
+        else Ei = QD::q(1.0, r.e + P);
+        r.ut = (double)QD::sqrt_island(f32_fabs((float)((m.M0 + P) * Ei)));
+        if constexpr (FAST) E2 = Ei * QuotFast::rcp1(r.ut);
+        else E2 = QD::q(Ei, r.ut);
+    }
     r.ux = m.M1 * E2;
     r.uy = m.M2 * E2;
     r.un = m.M3 * E2;
@@ -485,10 +663,41 @@ __device__ __forceinline__ Prim recover_finish(const EosDev &E, const Moments &m
     return r;
 }
 
+// getInferredVariables of N states sharing ePrev with DivTry: the values of
+// recover_moments where nothing fails (div.fails() else, and nan is left to
+// the evaluation that follows).
+template <bool TABLE, int N>
+__device__ __forceinline__ void recover_try(const EosDev &E, const Moments (&m)[N], const double (&Pi)[N],
+                                            double ePrev, int &nan, DivTry &div, Prim (&out)[N]) {
+    double e[N];
+    if (ePrev <= 0.1) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            e[k] = m[k].M0 - div_mid(m[k].M, m[k].M0);
+            div.ok = div.ok && in_range<-100, 100>(m[k].M0);
+        }
+    } else if constexpr (TABLE) {
+        table_roots_try<N>(E, ePrev, m, Pi, e, div.ok);
+    } else {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            int dummy = NAN_NONE;
+            e[k] = energy_from_conserved<false>(E, ePrev, m[k].M0, m[k].M, Pi[k], dummy);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) out[k] = recover_finish<TABLE, DivTry, QuotExact>(E, m[k], e[k], Pi[k], nan, div);
+}
+
 // getInferredVariables from the moments of the conserved variables.
 template <bool TABLE, class DV, class QD = QuotExact>
 __device__ __forceinline__ Prim recover_moments(const EosDev &E, const Moments &m, double Pi, double ePrev, int &nan,
                                                 DV &div) {
+    if constexpr (std::is_same_v<DV, DivTry>) {
+        Prim w[1];
+        recover_try<TABLE, 1>(E, {m}, {Pi}, ePrev, nan, div, w);
+        return w[0];
+    }
     double e;
     if (ePrev <= 0.1) {
         if constexpr (std::is_same_v<QD, QuotFast>) e = m.M0 - m.M * QuotFast::rcp1(m.M0);
@@ -505,6 +714,21 @@ __device__ __forceinline__ Prim recover(const EosDev &E, double t, double ttt, d
                                         int &nan, DV &div) {
     const Moments m = moments(t, ttt, ttx, tty, ttn, pitt, pitx, pity, pitn);
     return recover_moments<TABLE, DV, QD>(E, m, Pi, ePrev, nan, div);
+}
+
+// recover_moments with the division operator, for the cells whose DivTry
+// recovery fails; out of line (see role_terms_slow).
+struct RecoverSlow {
+    Prim w;
+    int nan;
+};
+template <bool TABLE>
+__device__ __attribute__((noinline)) RecoverSlow recover_slow(const void *eos, Moments m, double Pi, double ePrev) {
+    RecoverSlow r;
+    r.nan = NAN_NONE;
+    DivFast div;
+    r.w = recover_moments<TABLE>(*(const EosDev *)eos, m, Pi, ePrev, r.nan, div);
+    return r;
 }
 
 // Four root solves from one start value, stepped together: the table-EoS
@@ -567,6 +791,10 @@ __device__ __forceinline__ void recover4(const EosDev &E, double t, const double
         m[k] = moments(t, x[k][0], x[k][1], x[k][2], x[k][3], x[k][4], x[k][5], x[k][6], x[k][7]);
         Pi[k] = x[k][8];
         rn[k] = NAN_NONE;
+    }
+    if constexpr (std::is_same_v<DV, DivTry>) {
+        recover_try<TABLE, 4>(E, m, Pi, ePrev, nan, div, out);
+        return;
     }
     if (ePrev <= 0.1) {
 #pragma unroll

@@ -417,8 +417,8 @@ __global__ __launch_bounds__(64) void advance_clocks_kernel(EvDesc *__restrict__
 }
 
 // getInferredVariables (rhic/src/EnergyMomentumTensor.cpp:117-233) on
-// independent states, one thread each, through the same recover() the stage
-// kernel applies to its cell.
+// independent states, one thread each, through the same recovery the stage kernel
+// applies to its cell.
 template <bool TABLE>
 __global__ __launch_bounds__(256) void inferred_kernel(const EosDev E, int nc, double t, const double *__restrict__ q,
                                                        const double *__restrict__ ePrev, long n,
@@ -429,9 +429,15 @@ __global__ __launch_bounds__(256) void inferred_kernel(const EosDev E, int nc, d
 #pragma unroll
     for (int k = 0; k < 8; ++k) c[k] = q[k * n + i];
     const double Pi = nc == 15 ? q[14 * n + i] : 0.0;
-    DivFast div;
     int nan = NAN_NONE;
-    const Prim w = recover<TABLE>(E, t, c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], Pi, ePrev[i], nan, div);
+    const Moments m = moments(t, c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7]);
+    DivTry div;
+    Prim w = recover_moments<TABLE>(E, m, Pi, ePrev[i], nan, div);
+    if (div.fails()) {
+        const RecoverSlow r = recover_slow<TABLE>((const void *)__builtin_amdgcn_kernarg_segment_ptr(), m, Pi, ePrev[i]);
+        w = r.w;
+        nan = r.nan;
+    }
     out[i] = w.e;
     out[n + i] = w.p;
     out[2 * n + i] = w.ut;

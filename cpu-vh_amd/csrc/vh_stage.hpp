@@ -142,11 +142,6 @@ __device__ __forceinline__ double face_var_flux(const Side &R, const Side &L, do
     return res;
 }
 
-template <int DIR>
-__device__ __forceinline__ Side make_side(const Prim &w) {
-    return Side{DIR == 0 ? w.ux : (DIR == 1 ? w.uy : w.un), make_recip(w.ut)};
-}
-
 // The three limited slopes of one variable on the 5-point line
 // (qmm, qm, q, qp, qpp): D(qmm,qm,q), D(qm,q,qp), D(q,qp,qpp).  The four
 // half-site values of the two faces follow from them exactly as
@@ -183,8 +178,8 @@ __device__ __forceinline__ int pi_a_mu(int dir, int mu) {
 // is instantiated once.
 template <int NC, bool TABLE, class DV, class SINK, class GEO>
 __device__ __forceinline__ void dir_contrib(const StageParams &P, const GEO &G, const EosDev &E, long s, int dir, int coord,
-                                            int ncoord, long stride, double ePrev, double t, const Recip &rt2pow,
-                                            const Recip &rut, double v_c, SINK &&sink, int &nan, DV &div) {
+                                            int ncoord, long stride, double ePrev, double t, double t2pow,
+                                            double ut, double v_c, SINK &&sink, int &nan, DV &div) {
     auto nb = [&](int o) -> long {
         int c = coord + o;
         c = c < 0 ? 0 : (c >= ncoord ? ncoord - 1 : c);
@@ -192,7 +187,7 @@ __device__ __forceinline__ void dir_contrib(const StageParams &P, const GEO &G, 
     };
     const long sm2 = nb(-2), sm1 = nb(-1), sp1 = nb(1), sp2 = nb(2);
     const double d = dir == 0 ? G.dx : (dir == 1 ? G.dy : G.dz);
-    const Recip rd = make_recip(d);
+    const Recip rd = div.recip(d), rut = div.recip(ut);
 
     // Half-site values of the recovery inputs (q[0..7], Pi) on both faces.
     double qRf[9], qLf[9], qRb[9], qLb[9];
@@ -219,7 +214,7 @@ __device__ __forceinline__ void dir_contrib(const StageParams &P, const GEO &G, 
         Prim w[4];
         recover4<TABLE>(E, t, x, ePrev, nan, div, w);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) sd[q] = Side{dir == 0 ? w[q].ux : (dir == 1 ? w[q].uy : w[q].un), make_recip(w[q].ut)};
+        for (int q = 0; q < 4; ++q) sd[q] = Side{dir == 0 ? w[q].ux : (dir == 1 ? w[q].uy : w[q].un), div.recip(w[q].ut)};
     }
     const Side Rf = sd[0], Lf = sd[1], Rb = sd[2], Lb = sd[3];
     const double af = face_speed(Rf, Lf, div), ab = face_speed(Rb, Lb, div);
@@ -235,7 +230,7 @@ __device__ __forceinline__ void dir_contrib(const StageParams &P, const GEO &G, 
         const double dPi = dq(14);
         S[0] = S[0] - v * dPi;
         // S[a] -= dPi, with dPi / pow(t,2) along eta (SourceTerms.cpp:345,380,415)
-        const double dPa = dir == 2 ? div(dPi, rt2pow) : dPi;
+        const double dPa = dir == 2 ? div(dPi, div.recip(t2pow)) : dPi;
 #pragma unroll
         for (int mu = 1; mu < 4; ++mu)
             if (mu == dir + 1) S[mu] = S[mu] - dPa;
@@ -265,10 +260,10 @@ __device__ __forceinline__ void dir_contrib(const StageParams &P, const GEO &G, 
 // across the whole evaluation.
 template <int NC, bool TABLE, class DV, class GEO, class SINK>
 __device__ __forceinline__ void source_init(const StageParams &P, const GEO &G, const EosDev &E, long s, int i, int j, int k,
-                                            double t, const Recip &rt2pow, const Recip &rut, double ecell,
+                                            double t, double t2pow, double ut, double ecell,
                                             SINK &&sink, DV &div) {
-    const Recip rdx = make_recip(G.dx), rdy = make_recip(G.dy), rdz = make_recip(G.dz);
-    const Recip rt = make_recip(t), rdt = make_recip(G.dt);
+    const Recip rdx = div.recip(G.dx), rdy = div.recip(G.dy), rdz = div.recip(G.dz);
+    const Recip rt = div.recip(t), rdt = div.recip(G.dt), rt2pow = div.recip(t2pow), rut = div.recip(ut);
     const Recip r3{3.0, 1.0 / 3.0, true}, r5{5.0, 1.0 / 5.0, true};
     auto put = [&](int n, double Sn) { sink(n, P.q[n][s] + G.dt * Sn); };
     const double ttt = P.q[0][s], ttx = P.q[1][s], tty = P.q[2][s], ttn = P.q[3][s];
@@ -281,7 +276,7 @@ __device__ __forceinline__ void source_init(const StageParams &P, const GEO &G, 
     const double *__restrict__ unv = P.u[3];
     const double *__restrict__ pv = P.p;
     const double p = pv[s];
-    const double ut = utv[s], ux = uxv[s], uy = uyv[s], un = unv[s];
+    const double ux = uxv[s], uy = uyv[s], un = unv[s];
     const double utp = P.up[0][s], uxp = P.up[1][s], uyp = P.up[2][s], unp = P.up[3][s];
     const long strY = G.nx, strZ = (long)G.nx * G.ny;
     const long sl = i > 0 ? s - 1 : s, sr = i < G.nx - 1 ? s + 1 : s;
@@ -348,7 +343,7 @@ __device__ __forceinline__ void source_init(const StageParams &P, const GEO &G, 
         }
     }
     const double ut2 = ut * ut, un2 = un * un, t2 = t * t, t3 = t * t2;
-    const Recip rt2 = make_recip(t2), rt3 = make_recip(t3), r2t = make_recip(2.0 * t);
+    const Recip rt2 = div.recip(t2), rt3 = div.recip(t3), r2t = div.recip(2.0 * t);
         const double dtut = div(ut - utp, rdt);
     const double dtux = div(ux - uxp, rdt);
     const double dtuy = div(uy - uyp, rdt);
@@ -602,6 +597,50 @@ __device__ __forceinline__ StepTimes step_times(const StageParams &P, const EvDe
     return G.tab[G.base + P.off];
 }
 
+// One role's terms of cell s, variable n at out[n * CELLS_PER_BLOCK].
+template <int NC, bool TABLE, class DV, class GEO>
+__device__ __forceinline__ void role_terms(const StageParams &P, const GEO &G, const EosDev &E, long s, int i, int j,
+                                           int k, int role, double t, double t2pow, double *out, int &nan, DV &div) {
+    const double ecell = P.e[s], ut = P.u[0][s];
+    auto put = [&](int n, double a) {
+        div.see(a);
+        out[n * CELLS_PER_BLOCK] = a;
+    };
+    if (role == 0) {
+        div.in(ecell < 0x1p100);
+        source_init<NC, TABLE>(P, G, E, s, i, j, k, t, t2pow, ut, ecell, put, div);
+    } else {
+        const int dir = role - 1;
+        const int coord = dir == 0 ? i : (dir == 1 ? j : k);
+        const int ncoord = dir == 0 ? G.nx : (dir == 1 ? G.ny : G.nz);
+        const long stride = dir == 0 ? 1 : (dir == 1 ? (long)G.nx : (long)G.nx * G.ny);
+        dir_contrib<NC, TABLE>(P, G, E, s, dir, coord, ncoord, stride, ecell, t, t2pow, ut, P.u[1 + dir][s], put, nan,
+                               div);
+    }
+}
+
+// role_terms with DivFast, for the cells whose DivTry evaluation fails.  Kept
+// out of line: inlined, its register needs spill the common path's (70 VGPRs
+// against 2) and its code sits between the common path's.  The kernel's
+// parameters are read through the kernel argument segment (StageParams, then
+// EosDev), as taking their addresses would copy them to scratch on every
+// call; geo is the event's descriptor, or null where the parameters hold it.
+template <int NC, bool TABLE>
+__device__ __attribute__((noinline)) int role_terms_slow(const void *args, const EvDesc *geo, long s, int i, int j,
+                                                         int k, int role, double t, double t2pow, double *out) {
+    const StageParams &P = *(const StageParams *)args;
+    const EosDev &E = *(const EosDev *)((const char *)args + sizeof(StageParams));
+    static_assert(sizeof(StageParams) % alignof(EosDev) == 0, "EosDev follows StageParams in the argument segment");
+    DivFast div;
+    int nan = NAN_NONE;
+    role = __builtin_amdgcn_readfirstlane(role);
+    if (geo) role_terms<NC, TABLE>(P, *geo, E, s, i, j, k, role, t, t2pow, out, nan, div);
+    else role_terms<NC, TABLE>(P, P, E, s, i, j, k, role, t, t2pow, out, nan, div);
+    return nan;
+}
+__device__ __forceinline__ const EvDesc *slow_geo(const StageParams &) { return nullptr; }
+__device__ __forceinline__ const EvDesc *slow_geo(const EvDesc &G) { return &G; }
+
 template <int NC, bool TABLE, bool DIM3, class GEO>
 __device__ __forceinline__ void stage_body(const StageParams &P, const EosDev &E, const GEO &G, long blk) {
     constexpr int ROLES = DIM3 ? 4 : 3;
@@ -623,23 +662,12 @@ __device__ __forceinline__ void stage_body(const StageParams &P, const EosDev &E
     const double t2pow = P.stage ? st.t2sq : st.t1sq;
     const double t_new = st.t2;
     if (valid) {
-        DivFast div;
         int nan = NAN_NONE;
-        const double ecell = P.e[s];
-        const Recip rut = make_recip(P.u[0][s]);
-        const Recip rt2pow = make_recip(t2pow);
-        if (role == 0) {
-            source_init<NC, TABLE>(P, G, E, s, i, j, k, t, rt2pow, rut, ecell,
-                                   [&](int n, double a) { part[0][n][lane] = a; }, div);
-        } else {
-            auto put = [&](int n, double r) { part[role][n][lane] = r; };
-            const int dir = role - 1;
-            const int coord = dir == 0 ? i : (dir == 1 ? j : k);
-            const int ncoord = dir == 0 ? G.nx : (dir == 1 ? G.ny : G.nz);
-            const long stride = dir == 0 ? 1 : (dir == 1 ? (long)G.nx : (long)G.nx * G.ny);
-            dir_contrib<NC, TABLE>(P, G, E, s, dir, coord, ncoord, stride, ecell, t, rt2pow, rut, P.u[1 + dir][s], put,
-                                   nan, div);
-        }
+        DivTry div;
+        role_terms<NC, TABLE>(P, G, E, s, i, j, k, role, t, t2pow, &part[role][0][lane], nan, div);
+        if (__builtin_expect(div.fails(), 0))
+            nan = role_terms_slow<NC, TABLE>((const void *)__builtin_amdgcn_kernarg_segment_ptr(), slow_geo(G), s, i, j,
+                                             k, role, t, t2pow, &part[role][0][lane]);
         flags[role][lane] = nan;
     }
     __syncthreads();
@@ -664,10 +692,17 @@ __device__ __forceinline__ void stage_body(const StageParams &P, const EosDev &E
             o.acc[n] /= 2;
         }
     }
-    DivFast div;
     int nan_cell = NAN_NONE;
-    o.w = recover<TABLE>(E, t_new, o.acc[0], o.acc[1], o.acc[2], o.acc[3], o.acc[4], o.acc[5], o.acc[6], o.acc[7],
-                         NC == 15 ? o.acc[NC - 1] : 0.0, P.e[s], nan_cell, div);
+    const Moments m = moments(t_new, o.acc[0], o.acc[1], o.acc[2], o.acc[3], o.acc[4], o.acc[5], o.acc[6], o.acc[7]);
+    const double Pi = NC == 15 ? o.acc[NC - 1] : 0.0;
+    DivTry div;
+    o.w = recover_moments<TABLE>(E, m, Pi, P.e[s], nan_cell, div);
+    if (__builtin_expect(div.fails(), 0)) {
+        const RecoverSlow r = recover_slow<TABLE>((const char *)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(StageParams),
+                                                  m, Pi, P.e[s]);
+        o.w = r.w;
+        nan_cell = r.nan;
+    }
     o.fs = regulate<NC>(G, t_new, o.acc, o.w, nan_cell, o.fb);
     store_cell<NC>(P, s, o, nan != NAN_NONE ? nan : nan_cell);
 }
