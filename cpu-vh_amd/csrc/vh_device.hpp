@@ -427,10 +427,18 @@ __device__ __forceinline__ double nr_step(const EosDev &E, double e0, double M0,
 // small to change f').  e0's reciprocal serves both quotients by e0.  The
 // iteration is about half the instructions of the operator's, which spends
 // eleven on each of ten divisions and some twenty on the double square root.
-__device__ __forceinline__ double nr_step_try(const EosDev &E, double e0, double M0, double B, double Pi, DivTry &dx,
-                                              bool &ok) {
+// CS: how c_s^2 is found (eos_cs2): 0 it is 1/3, 1 delta_p/delta_e, 2 the reference's delta_e/delta_p.
+template <int CS>
+__device__ __forceinline__ double nr_step_try(const EosDev &E, double e0, double M0, double B, double Pi, bool &ok) {
+    DivTry dx;
     const double p = eos_pressure<true>(E, e0, dx);
-    const double cs2 = eos_cs2<true>(E, e0, dx);
+    double cs2 = 1. / 3.;
+    if constexpr (CS != 0) {
+        const double delta_p = eos_pressure<true>(E, e0 + E.e_spacing, dx) - p;
+        double v = CS == 1 ? div_mid(delta_p, E.e_spacing, E.r_spacing) : E.e_spacing / delta_p;
+        v = cs2 < v ? cs2 : v;
+        cs2 = 0.01 < v ? v : 0.01;
+    }
     const double r0 = near_rcp(e0);
     const double cst2 = div_mid(p, e0, r0);
     const double A = M0 * (1.0 - cst2) + Pi;
@@ -505,16 +513,20 @@ __device__ __forceinline__ RootResult table_root(const EosDev &E, double ePrev, 
 }
 
 // Table-EoS root solves from one start value, stepped together: table_root of
-// each state with nr_step_try.  Each takes exactly the steps table_root takes;
-// the N independent chains overlap.  A state that leaves nr_step_try's range
-// (a NaN among the causes), or has not converged after TRY_ITERS steps, ends
-// the attempt (ok false): the caller solves again with table_root, which
-// alone goes on to MAX_ITERS_NR and the bisection.
+// each state with nr_step_try.  Each takes exactly the steps table_root takes
+// (a state that has converged keeps its value while the others go on); a step
+// of all N evaluates them side by side, so their table gathers and chains
+// overlap where one state's step after another's waited for each gather: 60
+// steps of 131x131x61 with their copies 117.5 -> 110.6 ms, 100 steps of
+// 147x129 6.49 -> 6.24 ms, 16 batched events 16.9 -> 16.1 ms (one box).  A
+// state that leaves nr_step_try's range (a NaN among the causes), or has not
+// converged after TRY_ITERS steps, ends the attempt (ok false): the caller
+// solves again with table_root, which alone goes on to MAX_ITERS_NR and the
+// bisection.
 constexpr int TRY_ITERS = 64;
-template <int N>
-__device__ __forceinline__ void table_roots_try(const EosDev &E, double ePrev, const Moments (&m)[N],
-                                                const double (&Pi)[N], double (&e)[N], bool &ok) {
-    DivTry dx;
+template <int CS, int N>
+__device__ __forceinline__ void roots_try(const EosDev &E, double ePrev, const Moments (&m)[N], const double (&Pi)[N],
+                                          double (&e)[N], bool &ok) {
     double B[N];
     bool done[N];
 #pragma unroll
@@ -528,17 +540,42 @@ __device__ __forceinline__ void table_roots_try(const EosDev &E, double ePrev, c
         any = false;
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            if (!done[k]) {
-                bool in;
-                const double en = nr_step_try(E, e[k], m[k].M0, B[k], Pi[k], dx, in);
-                done[k] = nr_converged<QuotExact>(en, e[k]);
-                e[k] = en;
-                if (!in) ok = false;
-                any = any || !(done[k] || !in);
-            }
+            bool in;
+            const double en = nr_step_try<CS>(E, e[k], m[k].M0, B[k], Pi[k], in);
+            const bool conv = nr_converged<QuotExact>(en, e[k]);
+            ok = ok && (in || done[k]);
+            e[k] = done[k] ? e[k] : en;
+            done[k] = done[k] || conv || !in;
+            any = any || !done[k];
         }
     }
     ok = ok && !any;
+}
+// Four states go two at a time (four at once keep too much live: the
+// 131x131x61 step takes 1.3 % longer).
+template <int CS, int N>
+__device__ __forceinline__ void roots_by_two(const EosDev &E, double ePrev, const Moments (&m)[N], const double (&Pi)[N],
+                                             double (&e)[N], bool &ok) {
+    if constexpr (N == 4) {
+#pragma unroll
+        for (int h = 0; h < 4; h += 2) {
+            const Moments mh[2] = {m[h], m[h + 1]};
+            const double Ph[2] = {Pi[h], Pi[h + 1]};
+            double eh[2];
+            roots_try<CS, 2>(E, ePrev, mh, Ph, eh, ok);
+            e[h] = eh[0];
+            e[h + 1] = eh[1];
+        }
+    } else {
+        roots_try<CS, N>(E, ePrev, m, Pi, e, ok);
+    }
+}
+template <int N>
+__device__ __forceinline__ void table_roots_try(const EosDev &E, double ePrev, const Moments (&m)[N],
+                                                const double (&Pi)[N], double (&e)[N], bool &ok) {
+    if (E.cs2_const) roots_by_two<0, N>(E, ePrev, m, Pi, e, ok);
+    else if (E.cs2_mode) roots_by_two<1, N>(E, ePrev, m, Pi, e, ok);
+    else roots_by_two<2, N>(E, ePrev, m, Pi, e, ok);
 }
 
 // The segment of E.p4 holding e (clamped to the table's ends, where its
