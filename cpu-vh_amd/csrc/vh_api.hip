@@ -19,6 +19,7 @@
 
 #include "../../include/cpuvh_amd.h"
 #include "vh_host_eos.hpp"
+#include "vh_hostcopy.hpp"
 #include "vh_kernels.hpp"
 
 using namespace vh;
@@ -40,6 +41,7 @@ struct vh_handle {
     double *regfac = nullptr;   // regFacShear output, allocated on first request
     double *regfacb = nullptr;  // regFacBulk output (bulk builds), likewise
     int *d_err = nullptr;
+    HostCopy host;  // pinned memory of the downloads and of the error words
     unsigned long long *d_count = nullptr;
     // freezeout slices
     double *fo_prev = nullptr, *fo_cur = nullptr;
@@ -182,10 +184,9 @@ vh_status enqueue_step(vh_handle *h, const StepTimes &st, const StepTimes *tab, 
 }
 
 vh_status check_err(vh_handle *h) {
-    int err[4] = {0, 0, 0, 0};
-    HIPCHK(hipMemcpyAsync(err, h->d_err, sizeof(int) * 3, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h->host.fetch_err(h->d_err, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    return err[0] ? VH_ERR_NAN : VH_OK;
+    return h->host.err()[0] ? VH_ERR_NAN : VH_OK;
 }
 
 }  // namespace
@@ -253,6 +254,7 @@ vh_status vh_create(const vh_config *cfg, vh_handle **out) {
     for (int s = 0; s < 2; ++s, ptr += N) h->p[s] = ptr;
     if (hipMalloc(&h->d_err, sizeof(int) * 4) != hipSuccess) return fail(VH_ERR_NOMEM);
     if (hipMemset(h->d_err, 0, sizeof(int) * 4) != hipSuccess) return fail(VH_ERR_HIP);
+    if (h->host.init(N) != hipSuccess) return fail(VH_ERR_NOMEM);
     if (hipMalloc(&h->d_count, sizeof(unsigned long long)) != hipSuccess) return fail(VH_ERR_NOMEM);
     if (hipMalloc(&h->d_base, sizeof(int)) != hipSuccess) return fail(VH_ERR_NOMEM);
     if (hipHostMalloc(&h->h_base, sizeof(int), hipHostMallocDefault) != hipSuccess) return fail(VH_ERR_NOMEM);
@@ -282,6 +284,7 @@ vh_status vh_destroy(vh_handle *h) {
     hipFree(h->d_count);
     hipFree(h->d_base);
     if (h->h_base) hipHostFree(h->h_base);
+    h->host.release();
     hipFree(h->fo_prev);
     hipFree(h->fo_cur);
     hipFree(h->fo_ids);
@@ -516,8 +519,12 @@ vh_status vh_download(vh_handle *h, int field, double *out) {
     }
     double *src = field_ptr(h, field);
     if (!src) return VH_ERR_ARG;
-    HIPCHK(hipMemcpyAsync(out, src, sizeof(double) * h->N, hipMemcpyDeviceToHost, h->stream));
-    return check_err(h);
+    if (HostCopy::registered(out)) {
+        HIPCHK(hipMemcpyAsync(out, src, sizeof(double) * h->N, hipMemcpyDeviceToHost, h->stream));
+        return check_err(h);
+    }
+    HIPCHK(h->host.fetch(out, src, h->N, h->d_err, h->stream));
+    return h->host.err()[0] ? VH_ERR_NAN : VH_OK;
 }
 
 vh_status vh_thermal_vorticity(vh_handle *h) {

@@ -21,6 +21,7 @@
 
 #include "../../include/cpuvh_amd.h"
 #include "vh_host_eos.hpp"
+#include "vh_hostcopy.hpp"
 #include "vh_kernels.hpp"
 #include "vh_mixed.hpp"
 
@@ -77,6 +78,7 @@ struct vh_batch {
     HostEos heos;
     DeviceEos deos;
     int *d_err = nullptr;
+    HostCopy host;  // pinned memory of the downloads and of the error words
     std::vector<Event> ev;
     FoSurfaceWork fo_surf;  // vh_batch_fo_surface's device buffers
     std::map<long, long> free_seg;  // offset -> length
@@ -411,6 +413,7 @@ vh_status vh_batch_create(const vh_batch_config *cfg, vh_batch **out) {
     }
     if (hipMalloc(&b->d_err, sizeof(int) * 4) != hipSuccess || hipMemset(b->d_err, 0, sizeof(int) * 4) != hipSuccess)
         return fail(VH_ERR_NOMEM);
+    if (b->host.init(b->cap) != hipSuccess) return fail(VH_ERR_NOMEM);
     if (hipMalloc(&b->d_ev, sizeof(EvDesc) * c.max_events) != hipSuccess) return fail(VH_ERR_NOMEM);
     if (hipMalloc(&b->d_counts, sizeof(unsigned long long) * c.max_events) != hipSuccess) return fail(VH_ERR_NOMEM);
     if (hipMalloc(&b->d_strikes, sizeof(int) * c.max_events) != hipSuccess ||
@@ -450,6 +453,7 @@ vh_status vh_batch_destroy(vh_batch *b) {
     (void)hipFree(b->pool);
     (void)hipFree(b->fpool);
     (void)hipFree(b->stage_buf);
+    b->host.release();
     for (auto &H : b->hslot) {
         (void)hipHostFree(H.h);
         if (H.done) (void)hipEventDestroy(H.done);
@@ -799,19 +803,23 @@ vh_status vh_batch_run(vh_batch *b, double eF, int coarse, int nchecks, int32_t 
     return st;
 }
 
-vh_status vh_batch_sync(vh_batch *b) {
-    if (!b) return VH_ERR_ARG;
-    BCHK(hipSetDevice(b->dev));
-    int err[4] = {0, 0, 0, 0};
-    BCHK(hipMemcpyAsync(err, b->d_err, sizeof(int) * 3, hipMemcpyDeviceToHost, b->stream));
-    BCHK(hipStreamSynchronize(b->stream));
+// The status of work that has ended, the error words copied to b->host.
+static vh_status ended(vh_batch *b) {
     if (b->timed) {
         float ms = 0;
         BCHK(hipEventElapsedTime(&ms, b->ev0, b->ev1));
         b->last_ms = ms;
         b->timed = false;
     }
-    return err[0] ? VH_ERR_NAN : VH_OK;
+    return b->host.err()[0] ? VH_ERR_NAN : VH_OK;
+}
+
+vh_status vh_batch_sync(vh_batch *b) {
+    if (!b) return VH_ERR_ARG;
+    BCHK(hipSetDevice(b->dev));
+    BCHK(b->host.fetch_err(b->d_err, b->stream));
+    BCHK(hipStreamSynchronize(b->stream));
+    return ended(b);
 }
 
 double vh_batch_last_ms(const vh_batch *b) { return b ? b->last_ms : 0.0; }
@@ -844,8 +852,12 @@ vh_status vh_batch_download(vh_batch *b, int id, int field, double *out) {
     if (!b->mixed) {
         double *src = field_of(b, field, flip);
         if (!src) return VH_ERR_ARG;
-        BCHK(hipMemcpyAsync(out, src + E.off, sizeof(double) * E.N, hipMemcpyDeviceToHost, b->stream));
-        return vh_batch_sync(b);
+        if (HostCopy::registered(out)) {
+            BCHK(hipMemcpyAsync(out, src + E.off, sizeof(double) * E.N, hipMemcpyDeviceToHost, b->stream));
+            return vh_batch_sync(b);
+        }
+        BCHK(b->host.fetch(out, src + E.off, E.N, b->d_err, b->stream));
+        return ended(b);
     }
     const float *hi = nullptr, *lo = nullptr;
     if (!field_of_mixed(b, field, flip, &hi, &lo)) return VH_ERR_ARG;
@@ -853,6 +865,10 @@ vh_status vh_batch_download(vh_batch *b, int id, int field, double *out) {
     if (E.bi && (field == 3 || field == 7 || field == 10 || field == 12 || field == 20 || field == 24)) {
         std::fill(out, out + E.N, 0.0);
         return vh_batch_sync(b);
+    }
+    if (!HostCopy::registered(out)) {
+        BCHK(b->host.fetch_widened(out, hi + E.off, lo ? lo + E.off : nullptr, E.N, b->d_err, b->stream));
+        return ended(b);
     }
     double *tmp = nullptr;
     BCHK(hipMalloc(&tmp, sizeof(double) * E.N));

@@ -1,0 +1,106 @@
+// Device-to-host copies through pinned memory that its owner keeps.
+//
+// A download used to copy to the caller's pageable memory and then the error
+// word to a local variable, each a staged copy of the runtime with a wait of
+// its own, and in the mixed form allocated and freed a device buffer for the
+// widened values (a free waits for the whole device).  Here the field's
+// chunks and the error word go to pinned memory on the owner's stream, with
+// one wait for a field of one chunk; a longer field's chunks alternate between
+// two halves, one filled while the other is handed to the caller.  An FP32
+// field crosses as it is stored and is widened on the way out.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstring>
+
+namespace vh {
+
+class HostCopy {
+  public:
+    // Room for copies of at most largest doubles (longer ones go in chunks).
+    hipError_t init(size_t largest) {
+        half_ = std::min(MAX_HALF, std::max<size_t>(largest, 1));
+        hipError_t r = hipHostMalloc((void **)&buf_, 2 * half_ * sizeof(double) + ERR_BYTES, hipHostMallocDefault);
+        for (int k = 0; k < 2 && r == hipSuccess; ++k) r = hipEventCreateWithFlags(&full_[k], hipEventDisableTiming);
+        return r;
+    }
+    void release() {
+        if (buf_) (void)hipHostFree(buf_);
+        buf_ = nullptr;
+        for (auto &e : full_) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+    }
+    // Whether p is memory the runtime knows (pinned, managed, device): a copy
+    // there needs no staging, and the owners make it directly.
+    static bool registered(const void *p) {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        return a.type != hipMemoryTypeUnregistered;
+    }
+    // Pinned copy of the three error words, valid after the wait.
+    int *err() { return reinterpret_cast<int *>(buf_ + 2 * half_); }
+    hipError_t fetch_err(const int *d_err, hipStream_t st) {
+        return hipMemcpyAsync(err(), d_err, 3 * sizeof(int), hipMemcpyDeviceToHost, st);
+    }
+    // n doubles and the error words; waits.
+    hipError_t fetch(double *out, const double *src, size_t n, const int *d_err, hipStream_t st) {
+        return chunks(
+            n, d_err, st,
+            [&](double *b, size_t at, size_t len) {
+                return hipMemcpyAsync(b, src + at, len * sizeof(double), hipMemcpyDeviceToHost, st);
+            },
+            [&](const double *b, size_t at, size_t len) { std::memcpy(out + at, b, len * sizeof(double)); });
+    }
+    // n values hi (+ lo where not null), widened; waits.
+    hipError_t fetch_widened(double *out, const float *hi, const float *lo, size_t n, const int *d_err, hipStream_t st) {
+        return chunks(
+            n, d_err, st,
+            [&](double *b, size_t at, size_t len) {
+                float *f = reinterpret_cast<float *>(b);
+                hipError_t r = hipMemcpyAsync(f, hi + at, len * sizeof(float), hipMemcpyDeviceToHost, st);
+                if (r == hipSuccess && lo)
+                    r = hipMemcpyAsync(f + len, lo + at, len * sizeof(float), hipMemcpyDeviceToHost, st);
+                return r;
+            },
+            [&](const double *b, size_t at, size_t len) {
+                const float *h = reinterpret_cast<const float *>(b), *l = h + len;
+                double *o = out + at;
+                if (lo)
+                    for (size_t i = 0; i < len; ++i) o[i] = (double)h[i] + (double)l[i];
+                else
+                    for (size_t i = 0; i < len; ++i) o[i] = (double)h[i];
+            });
+    }
+
+  private:
+    static constexpr size_t MAX_HALF = size_t(1) << 17;  // doubles: 1 MiB, within a core's L2
+    static constexpr size_t ERR_BYTES = 64;
+    template <class COPY, class TAKE>
+    hipError_t chunks(size_t n, const int *d_err, hipStream_t st, COPY &&copy, TAKE &&take) {
+        const size_t count = (n + half_ - 1) / half_;
+        auto start = [&](size_t c) {
+            hipError_t r = copy(buf_ + (c & 1) * half_, c * half_, std::min(half_, n - c * half_));
+            if (r == hipSuccess && c + 1 == count) r = fetch_err(d_err, st);
+            return r == hipSuccess ? hipEventRecord(full_[c & 1], st) : r;
+        };
+        hipError_t r = start(0);
+        for (size_t c = 0; c < count && r == hipSuccess; ++c) {
+            if (c + 1 < count) r = start(c + 1);
+            if (r == hipSuccess) r = hipEventSynchronize(full_[c & 1]);
+            if (r == hipSuccess) take(buf_ + (c & 1) * half_, c * half_, std::min(half_, n - c * half_));
+        }
+        if (r != hipSuccess) (void)hipStreamSynchronize(st);  // no copy still writes the buffer
+        return r;
+    }
+    double *buf_ = nullptr;
+    size_t half_ = 0;
+    hipEvent_t full_[2] = {};
+};
+
+}  // namespace vh
