@@ -72,8 +72,16 @@ hipError_t launch_mx(const mx::MxFields &F, const EosDev &E, const EvDesc *ev, c
     return hipGetLastError();
 }
 
-// Tile variants: the face list of a tile fills whole passes of 256 threads
-// closely (16x15: 511 faces, 240 cells; 6x6x6: 756 faces, 216 cells).
+// Tile variants: the faces of each direction fit one pass of 256 threads
+// closely (16x15: 255 + 256 faces, 240 cells; 16x4x3: 204 + 240 + 256 faces,
+// 192 cells, which are three whole waves).  Rows of 16 cells in 3+1D: the
+// kernel issues some 400 loads per cell and stage, each as many cache lines
+// as its 64 lanes touch rows, and a 6x6x6 tile's loads touch eleven or more
+// (its waves waited to issue 55 % of their cycles).  40 steps of 201x201x101
+// with admission and downloads: 6x6x6 150.9 ms, 8x8x3 125.7, 8x4x6 120.8,
+// 16x4x3 110.9, 16x3x4 109.0; four events of 60 to 111 cells a side, 41 deep,
+// 47.4, 37.4, 35.9, 33.7, 34.2 ms.  12x4x4 (116.5), 21x3x3 (121.6) and 10x5x4
+// lie between.  In 2+1D 21x11, 18x13 and 25x9 measured 5 % slower than 16x15.
 // bi: every event of the launch is a boost-invariant 2+1D event (the
 // kernels that neither load nor evolve the eta components).
 template <int NC, bool TABLE>
@@ -93,8 +101,8 @@ hipError_t launch_mx_tile(const mx::MxFields &F, const EosDev &E, bool dim3d, in
         }
     } else {
         switch (tile) {
-        case 0: return launch_mx<NC, TABLE, true, 6, 6, 6>(F, E, ev, blk_ev, blk_first, nblocks, st);
-        case 1: return launch_mx<NC, TABLE, true, 8, 8, 3>(F, E, ev, blk_ev, blk_first, nblocks, st);
+        case 0: return launch_mx<NC, TABLE, true, 16, 4, 3>(F, E, ev, blk_ev, blk_first, nblocks, st);
+        case 1: return launch_mx<NC, TABLE, true, 16, 3, 4>(F, E, ev, blk_ev, blk_first, nblocks, st);
         case 2: return launch_mx<NC, TABLE, true, 8, 4, 6>(F, E, ev, blk_ev, blk_first, nblocks, st);
         }
     }
@@ -104,7 +112,7 @@ hipError_t launch_mx_tile(const mx::MxFields &F, const EosDev &E, bool dim3d, in
 }  // namespace
 
 const int MIXED_TILES_2D[MIXED_NTILE][3] = {{16, 15, 1}, {32, 7, 1}, {64, 3, 1}};
-const int MIXED_TILES_3D[MIXED_NTILE][3] = {{6, 6, 6}, {8, 8, 3}, {8, 4, 6}};
+const int MIXED_TILES_3D[MIXED_NTILE][3] = {{16, 4, 3}, {16, 3, 4}, {8, 4, 6}};
 
 hipError_t launch_stage_mixed(const mx::MxFields &F, const EosDev &E, int nc, bool dim3d, int tile, bool bi,
                               const EvDesc *ev, const int *blk_ev, const int *blk_first, int nblocks, hipStream_t st) {
