@@ -226,6 +226,21 @@ def _ptr(a):
     return a.ctypes.data_as(ctypes.c_void_p) if a is not None else None
 
 
+def _fo_surface(call, what, cubes, dim):
+    """One surface call with room for two elements a flagged cube (a cube has
+    rarely more than one); the device builds the elements a second time only
+    where that was too small.  Returns (n, elements, vars)."""
+    cap, total = 2 * cubes + 16, ctypes.c_int64()
+    while True:
+        el = np.empty((cap, 2 * dim), dtype=np.float64)
+        var = np.empty((cap, 10), dtype=np.float64)
+        st = call(_ptr(el), _ptr(var), cap, ctypes.byref(total))
+        if st != VH_ERR_CAPACITY or total.value <= cap:
+            Hydro._check(st, what)
+            return total.value, el, var
+        cap = total.value
+
+
 class Hydro:
     """One lattice on one GPU (a vh_handle)."""
 
@@ -350,16 +365,9 @@ class Hydro:
             raise ValueError(f"fo_surface: {dim} cell widths")
         m = (self.cfg.nx - 1) * (self.cfg.ny - 1) * (nz - 1 if nz > 1 else 1)
         counts = np.zeros(max(m, 1), dtype=np.int32)
-        total = ctypes.c_int64()
-        st = _lib().vh_fo_surface(self.h, _ptr(w), _ptr(counts), None, None, 0, ctypes.byref(total))
-        if st != VH_ERR_CAPACITY:
-            self._check(st, "vh_fo_surface")
-        cap = max(total.value, 1)
-        el = np.empty((cap, 2 * dim), dtype=np.float64)
-        var = np.empty((cap, 10), dtype=np.float64)
-        self._check(_lib().vh_fo_surface(self.h, _ptr(w), _ptr(counts), _ptr(el), _ptr(var), cap,
-                                         ctypes.byref(total)), "vh_fo_surface")
-        n = total.value
+        n, el, var = _fo_surface(
+            lambda *out: _lib().vh_fo_surface(self.h, _ptr(w), _ptr(counts), *out), "vh_fo_surface",
+            getattr(self, "_fo_n", 0), dim)
         return counts[:getattr(self, "_fo_n", 0)].copy(), el[:n].copy(), var[:n].copy()
 
     def eos_energy_density(self, T):
@@ -520,16 +528,9 @@ class Batch:
         w = np.ascontiguousarray(widths, dtype=np.float64)
         nf = getattr(self, "_fo_n", {}).get(eid, 0)
         counts = np.zeros(max(nf, 1), dtype=np.int32)
-        total = ctypes.c_int64()
-        st = _lib().vh_batch_fo_surface(self.b, eid, _ptr(w), _ptr(counts), None, None, 0, ctypes.byref(total))
-        if st != VH_ERR_CAPACITY:
-            Hydro._check(st, "vh_batch_fo_surface")
-        cap = max(total.value, 1)
-        el = np.empty((cap, 2 * dim), dtype=np.float64)
-        var = np.empty((cap, 10), dtype=np.float64)
-        Hydro._check(_lib().vh_batch_fo_surface(self.b, eid, _ptr(w), _ptr(counts), _ptr(el), _ptr(var), cap,
-                                                ctypes.byref(total)), "vh_batch_fo_surface")
-        n = total.value
+        n, el, var = _fo_surface(
+            lambda *out: _lib().vh_batch_fo_surface(self.b, eid, _ptr(w), _ptr(counts), *out),
+            "vh_batch_fo_surface", nf, dim)
         return counts[:nf].copy(), el[:n].copy(), var[:n].copy()
 
     def fo_surfaces(self, eids, widths, caps=None):
