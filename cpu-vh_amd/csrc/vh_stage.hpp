@@ -224,29 +224,41 @@ __device__ __forceinline__ void dir_contrib(const StageParams &P, const GEO &G, 
     const Side Rf = sd[0], Lf = sd[1], Rb = sd[2], Lb = sd[3];
     const double af = face_speed(Rf, Lf, div), ab = face_speed(Rb, Lb, div);
 
-    // pi-gradient terms of T^{tau mu} (central differences, fac = 1/d/2)
+    // Per-variable fluxes of both faces, then r.  pi and Pi come first, so that
+    // the pi-gradient terms of T^{tau mu} (central differences, fac = 1/d/2)
+    // are formed from the same lines, without eighteen loads of their own (131x131x61,
+    // 60 steps with copies: 97.8 -> 96.0 ms; 45x37x23: 4.87 -> 4.78 ms).
     const double fac = 1 / d / 2;
-    auto dq = [&](int n) { return (P.q[n][sp1] - P.q[n][sm1]) * fac; };
     const double v = div(v_c, rut);
-    double S[4];
+    double dT[4], dA[4] = {}, dPi = 0.0, S[4];
+    Points next = load_line(P.q[4], sm2, sm1, s, sp1, sp2);
 #pragma unroll
-    for (int mu = 0; mu < 4; ++mu) S[mu] = dq(4 + mu) * v - dq(pi_a_mu(dir, mu));
-    if constexpr (NC == 15) {
-        const double dPi = dq(14);
-        S[0] = S[0] - v * dPi;
-        // S[a] -= dPi, with dPi / pow(t,2) along eta (SourceTerms.cpp:345,380,415)
-        const double dPa = dir == 2 ? div(dPi, div.recip(t2pow)) : dPi;
+    for (int q = 0; q < NC; ++q) {
+        const int n = q + 4 < NC ? q + 4 : q + 4 - NC, n1 = n + 1 < NC ? n + 1 : 0;
+        const Points now = next;
+        if (q + 1 < NC) next = load_line(P.q[n1], sm2, sm1, s, sp1, sp2);
+        if (n >= 4) {
+            const double dq = (now.p - now.m) * fac;
+            if (n < 8) dT[n - 4] = dq;
 #pragma unroll
-        for (int mu = 1; mu < 4; ++mu)
-            if (mu == dir + 1) S[mu] = S[mu] - dPa;
-    }
-
-    // Per-variable fluxes of both faces, then r.
-    Points next = load_line(P.q[0], sm2, sm1, s, sp1, sp2);
+            for (int mu = 0; mu < 4; ++mu)
+                if (n == pi_a_mu(0, mu) || n == pi_a_mu(1, mu) || n == pi_a_mu(2, mu))
+                    dA[mu] = n == pi_a_mu(dir, mu) ? dq : dA[mu];
+            if (n == 14) dPi = dq;
+        }
+        if (n == 0) {
 #pragma unroll
-    for (int n = 0; n < NC; ++n) {
-        const Line l = make_line(next);
-        if (n + 1 < NC) next = load_line(P.q[n + 1], sm2, sm1, s, sp1, sp2);
+            for (int mu = 0; mu < 4; ++mu) S[mu] = dT[mu] * v - dA[mu];
+            if constexpr (NC == 15) {
+                S[0] = S[0] - v * dPi;
+                // S[a] -= dPi, with dPi / pow(t,2) along eta (SourceTerms.cpp:345,380,415)
+                const double dPa = dir == 2 ? div(dPi, div.recip(t2pow)) : dPi;
+#pragma unroll
+                for (int mu = 1; mu < 4; ++mu)
+                    if (mu == dir + 1) S[mu] = S[mu] - dPa;
+            }
+        }
+        const Line l = make_line(now);
         const double Hf = face_var_flux(Rf, Lf, af, right_fwd(l), left_fwd(l), div);
         const double Hb = face_var_flux(Rb, Lb, ab, right_bwd(l), left_bwd(l), div);
         double r = -Hf;
