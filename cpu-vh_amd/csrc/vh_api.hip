@@ -601,7 +601,7 @@ vh_status vh_fo_flag(vh_handle *h, double eF, int64_t *ids, double *corners, int
         HIPCHK(hipMalloc(&h->fo_prev, b));
         HIPCHK(hipMalloc(&h->fo_cur, b));
         // the ids, then the flag kernels' per-block scratch
-        HIPCHK(hipMalloc(&h->fo_ids, sizeof(long long) * (std::max(1L, M) + fo_flag_blocks(M))));
+        HIPCHK(hipMalloc(&h->fo_ids, sizeof(long long) * (std::max(1L, M) + fo_flag_scratch(M))));
         HIPCHK(hipMemsetAsync(h->fo_prev, 0, b, h->stream));  // calloc'd slices, HydroPlugin.cpp:159
         HIPCHK(hipMemsetAsync(h->fo_cur, 0, b, h->stream));
     }

@@ -916,7 +916,7 @@ static vh_status fo_flag_enqueue(vh_batch *b, int id, double eF, unsigned long l
         BCHK(hipMalloc(&E.fo_prev, bytes));
         BCHK(hipMalloc(&E.fo_cur, bytes));
         // the ids, then the flag kernels' per-block scratch
-        BCHK(hipMalloc(&E.fo_ids, sizeof(long long) * (std::max(1L, M) + fo_flag_blocks(M))));
+        BCHK(hipMalloc(&E.fo_ids, sizeof(long long) * (std::max(1L, M) + fo_flag_scratch(M))));
         BCHK(hipMemsetAsync(E.fo_prev, 0, bytes, b->stream));
         BCHK(hipMemsetAsync(E.fo_cur, 0, bytes, b->stream));
     }

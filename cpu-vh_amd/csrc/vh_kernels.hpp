@@ -56,8 +56,10 @@ hipError_t launch_admit_fp64(const AdmitSrc &S, double *q, double *e0, double *p
                              long N, long off, int nc, int *strikes, int *stop, hipStream_t st);
 hipError_t launch_count_above(const double *e, long N, double eF, unsigned long long *out, hipStream_t st);
 // The cut cubes' ids in increasing order into ids (capacity cap), their
-// number into *count; blk is scratch of fo_flag_blocks(cubes) entries.
-inline long fo_flag_blocks(long cubes) { return (cubes + 255) / 256; }
+// number into *count; blk is scratch of fo_flag_scratch(cubes) entries: the
+// count, then the offset, of each block of 256 cubes, and its four waves' masks.
+inline constexpr long fo_flag_blocks(long cubes) { return (cubes + 255) / 256; }
+inline constexpr long fo_flag_scratch(long cubes) { return 5 * fo_flag_blocks(cubes); }
 hipError_t launch_fo_flag(const double *eprev, const double *ecur, int nx, int ny, int nz, double eF,
                           long long *ids, long long cap, unsigned long long *count, unsigned long long *blk,
                           hipStream_t st);

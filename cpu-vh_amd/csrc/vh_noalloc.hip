@@ -1,6 +1,6 @@
 // vh_fo_flag_noalloc: the freezeout crossing test and ordered compaction of
 // vh_fo_flag on caller-owned device slices, with the kernels' per-block
-// counts in a fixed device array of the library instead of memory allocated
+// counts and masks in a fixed device array of the library instead of memory allocated
 // per call, so that callers which cannot allocate (code under HIP graph
 // capture, tight serving loops) can flag cubes.  No counterpart in the
 // reference.
@@ -14,12 +14,12 @@
 
 namespace {
 
-constexpr long MAX_BLOCKS = VH_FO_NOALLOC_MAX_CUBES / 256;
+constexpr long MAX_SCRATCH = vh::fo_flag_scratch(VH_FO_NOALLOC_MAX_CUBES);
 constexpr int MAX_DEVICES = 64;
 
-// per-block counts of the flag kernels (fo_flag_blocks(M) entries); each GPU
+// per-block counts and masks of the flag kernels (2.5 MiB); each GPU
 // holds its own copy until the process ends
-static __device__ __align__(256) unsigned long long scratch[MAX_BLOCKS];
+static __device__ __align__(256) unsigned long long scratch[MAX_SCRATCH];
 
 std::mutex g_mu;
 unsigned long long *g_scratch[MAX_DEVICES] = {};  // device address of scratch, per device

@@ -205,7 +205,7 @@ vh_status vh_fo_surface(vh_handle *h, const double *widths, int *n_el, double *e
  * hipStream_t, NULL for the null stream) of the current device, with no
  * synchronisation, so the call can be captured into a graph; the results are
  * there once the stream reaches them.  The kernels' per-block counts live in
- * one fixed device array of the library per GPU (512 KiB, kept until the
+ * one fixed device array of the library per GPU (2.5 MiB, kept until the
  * process ends): at most VH_FO_NOALLOC_MAX_CUBES cubes ((nx-1)(ny-1)(nz-1),
  * nz-1 read as 1 in 2+1D), else VH_ERR_ARG; calls that overlap on one GPU race
  * for that array. */
