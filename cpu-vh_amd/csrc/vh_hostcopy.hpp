@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 
 namespace vh {
 
@@ -83,6 +84,7 @@ class HostCopy {
     static constexpr size_t ERR_BYTES = 64;
     template <class COPY, class TAKE>
     hipError_t chunks(size_t n, const int *d_err, hipStream_t st, COPY &&copy, TAKE &&take) {
+        std::lock_guard<std::mutex> lock(mu_);  // downloads of one owner from two threads take turns
         const size_t count = (n + half_ - 1) / half_;
         auto start = [&](size_t c) {
             hipError_t r = copy(buf_ + (c & 1) * half_, c * half_, std::min(half_, n - c * half_));
@@ -98,6 +100,7 @@ class HostCopy {
         if (r != hipSuccess) (void)hipStreamSynchronize(st);  // no copy still writes the buffer
         return r;
     }
+    std::mutex mu_;
     double *buf_ = nullptr;
     size_t half_ = 0;
     hipEvent_t full_[2] = {};
