@@ -179,8 +179,8 @@ __device__ __forceinline__ int pi_a_mu(int dir, int mu) {
 // variable by variable: r = ((-H_{+1/2} + H_{-1/2}) / d [+ S_d]) * dt.  dir
 // is wave-uniform, so the three directions share one body.  Every face flux
 // uses the owning cell's e as the root solve's previous value, as the
-// reference does; the four half-site root solves run in a loop so the solver
-// is instantiated once.
+// reference does; the four half-site root solves go two at a time
+// (roots_by_two).
 template <int NC, bool TABLE, class DV, class SINK, class GEO>
 __device__ __forceinline__ void dir_contrib(const StageParams &P, const GEO &G, const EosDev &E, long s, int dir, int coord,
                                             int ncoord, long stride, double ePrev, double t, double t2pow,
