@@ -177,11 +177,12 @@ __global__ __launch_bounds__(1024) void fo_flag_scan_kernel(unsigned long long *
 __global__ __launch_bounds__(256) void fo_flag_write_kernel(const unsigned long long *__restrict__ blk,
                                                             long long *__restrict__ ids, long long cap) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const unsigned long long *masks = blk + gridDim.x + blockIdx.x * 4ul;
-    const unsigned long long mask = masks[w];
+    const unsigned long long *m = blk + gridDim.x + blockIdx.x * 4ul;
+    const unsigned long long off = blk[blockIdx.x], m0 = m[0], m1 = m[1], m2 = m[2], m3 = m[3];  // one wait
+    const unsigned long long mask = w < 2 ? (w ? m1 : m0) : (w == 2 ? m2 : m3);
     if (!(mask >> lane & 1)) return;
-    unsigned long long pos = blk[blockIdx.x] + (unsigned long long)__popcll(mask & ((1ull << lane) - 1ull));
-    for (int k = 0; k < w; ++k) pos += (unsigned long long)__popcll(masks[k]);
+    unsigned long long pos = off + (unsigned long long)__popcll(mask & ((1ull << lane) - 1ull));
+    pos += (unsigned long long)((w > 0 ? __popcll(m0) : 0) + (w > 1 ? __popcll(m1) : 0) + (w > 2 ? __popcll(m2) : 0));
     if ((long long)pos < cap) ids[pos] = (long long)blockIdx.x * 256 + threadIdx.x;
 }
 
