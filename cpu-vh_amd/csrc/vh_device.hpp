@@ -88,28 +88,46 @@ struct DivExact {
 // |b| in [2^-300, 2^300], or a zero.  The residual is taken as b q0 - a so
 // that a zero a keeps its sign for b > 0.  near_rcp(b) serves several
 // numerators of one divisor.
-__device__ __forceinline__ double near_rcp(double b) {
+__host__ __device__ __forceinline__ double near_rcp(double b) {
+#ifdef __HIP_DEVICE_COMPILE__
     double r = __builtin_amdgcn_rcp(b);
     r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
     return __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+#else
+    return 1.0 / b;  // host checks of the division policies
+#endif
 }
-__device__ __forceinline__ double div_mid(double a, double b, double r) {
+__host__ __device__ __forceinline__ double div_mid(double a, double b, double r) {
     const double q0 = a * r;
     const double rem = __builtin_fma(b, q0, -a);
     return __builtin_fma(-rem, r, q0);
 }
-__device__ __forceinline__ double div_mid(double a, double b) { return div_mid(a, b, near_rcp(b)); }
+__host__ __device__ __forceinline__ double div_mid(double a, double b) { return div_mid(a, b, near_rcp(b)); }
 
+__host__ __device__ __forceinline__ uint32_t high_word(double x) {
+    return (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32);
+}
 // The high word of |x| less that of 2^LO as an unsigned number lies below this
 // span exactly when 2^LO <= |x| < 2^HI; NaN, infinities, zeros and, for the
 // signed form, negative x fall outside.
 template <int LO, int HI>
-__device__ __forceinline__ bool in_range(double x) {
-    return (uint32_t)__double2hiint(x) - (uint32_t)((1023 + LO) << 20) < (uint32_t)((HI - LO) << 20);
+__host__ __device__ __forceinline__ bool in_range(double x) {
+    return high_word(x) - (uint32_t)((1023 + LO) << 20) < (uint32_t)((HI - LO) << 20);
 }
 template <int LO, int HI>
-__device__ __forceinline__ bool abs_in_range(double x) {
-    return ((uint32_t)__double2hiint(x) << 1) - ((uint32_t)(1023 + LO) << 21) < ((uint32_t)(HI - LO) << 21);
+__host__ __device__ __forceinline__ bool abs_in_range(double x) {
+    return (high_word(x) << 1) - ((uint32_t)(1023 + LO) << 21) < ((uint32_t)(HI - LO) << 21);
+}
+// x's exponent, |x| in [2^(k-1), 2^k), subnormal x included; 0 for zeros,
+// infinities and NaN.
+__host__ __device__ __forceinline__ int exponent(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_frexp_exp(x);
+#else
+    int k = 0;
+    if (__builtin_isfinite(x)) __builtin_frexp(x, &k);
+    return k;
+#endif
 }
 
 // sqrtf of a float x that is zero or >= 2^-96 (NaN and infinity keep their
@@ -129,43 +147,43 @@ __device__ __forceinline__ float sqrt_mid(float x) {
 // Division policy of the FP64 stage: every quotient by the reciprocal form,
 // unchecked, with what the check needs accumulated beside it.  The caller
 // asks fails() once at the end and, if some lane's operands left the range,
-// evaluates the whole expression again with DivFast.  What has to hold is
-// DivFast's condition: every divisor in [2^-16, 2^100], every quotient zero or
-// in [2^-950, ...) (then the residual is a multiple of 2^-1074 and exactly
-// representable), nothing overflowed; a quotient that overflows or is NaN
-// makes the results NaN or infinite, which see() notes.  Quotients below
-// 2^-1042 count as zero.  DivFast compares, selects and branches at each of
-// about 300 divisions a cell and stage (three 64-bit compares, a select and a
-// branch each); here a division costs its four instructions and one and a
-// half 32-bit ones.  With nr_step_try the 3+1D kernel issues 2.36e8 VALU
+// evaluates the whole expression again with DivFast.  What has to hold: every
+// divisor b in [2^-16, 2^50), every numerator a zero or |a| >= 2^-969, nothing
+// overflowed.  Then q0 is normal (at least 2^-1020) and the residual b q0 - a is
+// a multiple of 2^-1074, so it is exactly representable and the corrected
+// quotient is the division operator's; a == +-0 gives the correctly signed
+// zero.  The check is on a, not on q0: a subnormal quotient's high word can be
+// zero, as a zero's is, and a's exponent does not wait for the product.  A quotient that overflows or is NaN makes the results
+// NaN or infinite, which see() notes.  DivFast compares, selects and branches
+// at each of about 300 divisions a cell and stage (three 64-bit compares, a
+// select and a branch each); here a division costs its four instructions and
+// two 32-bit ones.  With nr_step_try the 3+1D kernel issues 2.36e8 VALU
 // instructions per launch at 131x131x61 where it issued 3.35e8; with their
 // copies, 60 steps of that event took 112.8 instead of 122.8 ms, 100 steps of
 // a 147x129 event 6.48 instead of 8.32 ms, 200 conformal steps at 201x201 9.87
 // instead of 12.2 ms, 40 steps of 16 batched events 16.6 instead of 18.9 ms.
 struct DivTry {
-    uint32_t lo = 0xffffffffu, hi = 0;
+    static constexpr int MIN_EXPONENT = -968;  // of a numerator that is not zero
+    int lo = 0;
+    uint32_t hi = 0;
     bool ok = true;
-    __device__ __forceinline__ Recip recip(double b) {
+    __host__ __device__ __forceinline__ Recip recip(double b) {
         double r = near_rcp(b);
         r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);  // 1/b correctly rounded
-        ok = ok && in_range<-16, 100>(b);
+        ok = ok && in_range<-16, 50>(b);
         return Recip{b, r, true};
     }
-    __device__ __forceinline__ double operator()(double a, const Recip &R) {
-        const double q0 = a * R.r;
-        const double rem = __builtin_fma(R.b, q0, -a);
-        const uint32_t u = ((uint32_t)__double2hiint(q0) << 1) + 0xffffffffu;  // zero becomes the largest
-        lo = u < lo ? u : lo;
-        return __builtin_fma(-rem, R.r, q0);
+    __host__ __device__ __forceinline__ double operator()(double a, const Recip &R) {
+        const int k = exponent(a);
+        lo = k < lo ? k : lo;
+        return div_mid(a, R.b, R.r);
     }
-    __device__ __forceinline__ void see(double x) {
-        const uint32_t u = (uint32_t)__double2hiint(x) << 1;
+    __host__ __device__ __forceinline__ void see(double x) {
+        const uint32_t u = high_word(x) << 1;
         hi = u > hi ? u : hi;
     }
-    __device__ __forceinline__ void in(bool inside) { ok = ok && inside; }
-    __device__ __forceinline__ bool fails() const {
-        return !ok || lo < ((1023u - 950u) << 21) - 1u || hi >= 0x7ffu << 21;
-    }
+    __host__ __device__ __forceinline__ void in(bool inside) { ok = ok && inside; }
+    __host__ __device__ __forceinline__ bool fails() const { return !ok || lo < MIN_EXPONENT || hi >= 0x7ffu << 21; }
 };
 // The table lookups of DivTry's callers: their quotients need no check (a
 // quotient too small for the residual to be exact changes neither the index

@@ -1,0 +1,64 @@
+// Host check of the FP64 stage's division policy (vh::DivTry): whatever it
+// accepts has the division operator's bits, and it accepts what it says it
+// does.  Prints one line per part, "mismatches M refused R of N".
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <random>
+
+#include "../cpu-vh_amd/csrc/vh_device.hpp"
+
+namespace {
+
+std::mt19937_64 rng(2024);
+
+// sign and mantissa at random (some mantissas all zeros or all ones), |x| in [2^k, 2^(k+1)), k >= -1074
+double make(int k, bool positive) {
+    uint64_t m = rng() & ((1ull << 52) - 1);
+    const unsigned pick = rng() & 15;
+    if (pick == 0) m = 0;
+    if (pick == 1) m = (1ull << 52) - 2;
+    uint64_t u;
+    if (k >= -1022) u = ((uint64_t)(k + 1023) << 52) | m;
+    else u = (1ull << (k + 1074)) | (m & ((1ull << (k + 1074)) - 1));
+    if (!positive && (rng() & 1)) u |= 1ull << 63;
+    double x;
+    std::memcpy(&x, &u, 8);
+    return x;
+}
+int between(int lo, int hi) { return lo + (int)(rng() % (uint64_t)(hi - lo + 1)); }
+
+bool same(double x, double y) { return std::memcmp(&x, &y, 8) == 0; }
+
+// numerators of exponents [alo, ahi], divisors of [blo, bhi]
+long part(const char *name, long n, int alo, int ahi, int blo, int bhi, bool all_accepted) {
+    long bad = 0, refused = 0;
+    for (long i = 0; i < n; ++i) {
+        const double a = alo > ahi ? (rng() & 1 ? 0.0 : -0.0) : make(between(alo, ahi), false);
+        const double b = make(between(blo, bhi), true);
+        vh::DivTry d;
+        const double q = d(a, d.recip(b));
+        d.see(q);
+        if (d.fails()) ++refused;
+        else if (!same(q, a / b)) ++bad;
+    }
+    const bool wrong = bad || (all_accepted && refused);
+    std::printf("%s: mismatches %ld refused %ld of %ld%s\n", name, bad, refused, n, wrong ? " WRONG" : "");
+    return wrong;
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+    const long n = argc > 1 ? std::atol(argv[1]) : 1000000;
+    long wrong = 0;
+    wrong += part("ordinary", n, -960, 800, -16, 49, true);
+    wrong += part("smallest accepted numerators", n, -969, -960, -16, 49, true);
+    wrong += part("zero numerators", n, 1, 0, -16, 49, true);
+    wrong += part("small numerators", n, -1000, -950, -16, 49, false);
+    wrong += part("subnormal quotients", n, -1074, -1000, -16, 49, false);
+    wrong += part("quotients of the last bits", n, -1074, -1060, -4, 8, false);
+    wrong += part("overflowing quotients", n, 1000, 1023, -16, 20, false);
+    wrong += part("divisors outside", n, -960, 800, -140, 140, false);
+    return wrong ? 1 : 0;
+}
