@@ -148,7 +148,7 @@ __device__ __forceinline__ float sqrt_mid(float x) {
 // unchecked, with what the check needs accumulated beside it.  The caller
 // asks fails() once at the end and, if some lane's operands left the range,
 // evaluates the whole expression again with DivFast.  What has to hold: every
-// divisor b in [2^-16, 2^50), every numerator a zero or |a| >= 2^-969, nothing
+// divisor b in [2^-100, 2^50), every numerator a zero or |a| >= 2^-969, nothing
 // overflowed.  Then q0 is normal (at least 2^-1020) and the residual b q0 - a is
 // a multiple of 2^-1074, so it is exactly representable and the corrected
 // quotient is the division operator's; a == +-0 gives the correctly signed
@@ -170,7 +170,7 @@ struct DivTry {
     __host__ __device__ __forceinline__ Recip recip(double b) {
         double r = near_rcp(b);
         r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);  // 1/b correctly rounded
-        ok = ok && in_range<-16, 50>(b);
+        ok = ok && in_range<-100, 50>(b);
         return Recip{b, r, true};
     }
     __host__ __device__ __forceinline__ double operator()(double a, const Recip &R) {

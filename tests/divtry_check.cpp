@@ -55,6 +55,8 @@ int main(int argc, char **argv) {
     wrong += part("ordinary", n, -960, 800, -16, 49, true);
     wrong += part("smallest accepted numerators", n, -969, -960, -16, 49, true);
     wrong += part("zero numerators", n, 1, 0, -16, 49, true);
+    // t^3 at t = 0.001, dt = 1e-9: the time's powers and the step are divisors too
+    wrong += part("small divisors", n, -900, 800, -100, -16, true);
     wrong += part("small numerators", n, -1000, -950, -16, 49, false);
     wrong += part("subnormal quotients", n, -1074, -1000, -16, 49, false);
     wrong += part("quotients of the last bits", n, -1074, -1060, -4, 8, false);

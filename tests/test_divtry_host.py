@@ -16,4 +16,4 @@ def test_accepted_quotients_are_the_operators(tmp_path):
                     "-o", exe, os.path.join(HERE, "divtry_check.cpp")], check=True, capture_output=True)
     r = subprocess.run([exe, "2000000"], capture_output=True, text=True, timeout=300)
     print(r.stdout)
-    assert r.returncode == 0 and r.stdout.count("mismatches 0") == 8, r.stdout
+    assert r.returncode == 0 and r.stdout.count("mismatches 0") == 9, r.stdout
