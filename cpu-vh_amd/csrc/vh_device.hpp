@@ -153,8 +153,12 @@ __device__ __forceinline__ float sqrt_mid(float x) {
 // a multiple of 2^-1074, so it is exactly representable and the corrected
 // quotient is the division operator's; a == +-0 gives the correctly signed
 // zero.  The check is on a, not on q0: a subnormal quotient's high word can be
-// zero, as a zero's is, and a's exponent does not wait for the product.  A quotient that overflows or is NaN makes the results
-// NaN or infinite, which see() notes.  DivFast compares, selects and branches
+// zero, as a zero's is, and a's exponent does not wait for the product.
+// Divisors reach down to 2^-100 because t, t^2, t^3 and dt are among them (with
+// a floor of 2^-16 every cell below t = 0.025 or dt = 1.5e-5 took the checked
+// evaluation: 40 steps of 61x57x31 at t = 0.001 and dt = 1e-5 took 11.3 ms
+// instead of 5.7).  A quotient that overflows or is NaN makes the results NaN
+// or infinite, which see() notes.  DivFast compares, selects and branches
 // at each of about 300 divisions a cell and stage (three 64-bit compares, a
 // select and a branch each); here a division costs its four instructions and
 // two 32-bit ones.  With nr_step_try the 3+1D kernel issues 2.36e8 VALU
