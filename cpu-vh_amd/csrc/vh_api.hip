@@ -620,8 +620,9 @@ vh_status vh_fo_flag(vh_handle *h, double eF, int64_t *ids, double *corners, int
                                   h->stream));
     }
     HIPCHK(hipMemsetAsync(h->d_count, 0, sizeof(unsigned long long), h->stream));
-    HIPCHK(launch_fo_flag(h->fo_prev, h->fo_cur, c.nx, c.ny, c.nz, eF, h->fo_ids, M, h->d_count,
-                          (unsigned long long *)(h->fo_ids + std::max(1L, M)), h->stream));
+    unsigned long long *blk = (unsigned long long *)(h->fo_ids + std::max(1L, M));
+    HIPCHK(launch_fo_flag(h->fo_prev, h->fo_cur, c.nx, c.ny, c.nz, eF, h->fo_ids, M, h->d_count, blk,
+                          blk + fo_flag_blocks(M), h->stream));
     unsigned long long n = 0;
     HIPCHK(hipMemcpyAsync(&n, h->d_count, sizeof(n), hipMemcpyDeviceToHost, h->stream));
     vh_status s = check_err(h);

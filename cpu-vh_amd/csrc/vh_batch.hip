@@ -951,8 +951,9 @@ static vh_status fo_flag_enqueue(vh_batch *b, int id, double eF, unsigned long l
         }
         if (b->mixed) BCHK(launch_widen_set(W, E.N, b->stream));
     }
-    BCHK(launch_fo_flag(E.fo_prev, E.fo_cur, c.nx, c.ny, c.nz, eF, E.fo_ids, M, count,
-                        (unsigned long long *)(E.fo_ids + std::max(1L, M)), b->stream));
+    unsigned long long *blk = (unsigned long long *)(E.fo_ids + std::max(1L, M));
+    BCHK(launch_fo_flag(E.fo_prev, E.fo_cur, c.nx, c.ny, c.nz, eF, E.fo_ids, M, count, blk, blk + fo_flag_blocks(M),
+                        b->stream));
     return VH_OK;
 }
 

@@ -131,14 +131,15 @@ __device__ __forceinline__ bool fo_cut(const double *__restrict__ eprev, const d
 // 131x131x61 among others, of which some 12 are the three launches.
 __global__ __launch_bounds__(256) void fo_flag_count_kernel(const double *__restrict__ eprev,
                                                             const double *__restrict__ ecur, int nx, int ny, int nz,
-                                                            double eF, long M, unsigned long long *__restrict__ blk) {
+                                                            double eF, long M, unsigned long long *__restrict__ blk,
+                                                            unsigned long long *__restrict__ masks) {
     __shared__ unsigned int part[4];
     const long c = (long)blockIdx.x * 256 + threadIdx.x;
     const bool flag = c < M && fo_cut(eprev, ecur, nx, ny, nz, eF, c);
     const unsigned long long mask = __ballot(flag);
     if ((threadIdx.x & 63) == 0) {
         part[threadIdx.x >> 6] = (unsigned int)__popcll(mask);
-        blk[gridDim.x + blockIdx.x * 4ul + (threadIdx.x >> 6)] = mask;
+        masks[blockIdx.x * 4ul + (threadIdx.x >> 6)] = mask;
     }
     __syncthreads();
     if (threadIdx.x == 0) blk[blockIdx.x] = (unsigned long long)part[0] + part[1] + part[2] + part[3];
@@ -175,15 +176,14 @@ __global__ __launch_bounds__(1024) void fo_flag_scan_kernel(unsigned long long *
 }
 
 __global__ __launch_bounds__(256) void fo_flag_write_kernel(const unsigned long long *__restrict__ blk,
+                                                            const unsigned long long *__restrict__ masks, long M,
                                                             long long *__restrict__ ids, long long cap) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const unsigned long long *m = blk + gridDim.x + blockIdx.x * 4ul;
-    const unsigned long long off = blk[blockIdx.x], m0 = m[0], m1 = m[1], m2 = m[2], m3 = m[3];  // one wait
-    const unsigned long long mask = w < 2 ? (w ? m1 : m0) : (w == 2 ? m2 : m3);
-    if (!(mask >> lane & 1)) return;
-    unsigned long long pos = off + (unsigned long long)__popcll(mask & ((1ull << lane) - 1ull));
-    pos += (unsigned long long)((w > 0 ? __popcll(m0) : 0) + (w > 1 ? __popcll(m1) : 0) + (w > 2 ? __popcll(m2) : 0));
-    if ((long long)pos < cap) ids[pos] = (long long)blockIdx.x * 256 + threadIdx.x;
+    const unsigned long long *b = masks + blockIdx.x * 4ul;
+    const unsigned long long off = blk[blockIdx.x], m0 = b[0], m1 = b[1], m2 = b[2], m3 = b[3];  // one wait
+    const long first = (long)blockIdx.x * 256;
+    const long long pos = fo_flag_place(off, m0, m1, m2, m3, w, lane, first, M, cap);
+    if (pos >= 0) ids[pos] = first + threadIdx.x;
 }
 
 // Corner energies of the flagged cubes for the host surface builder.
@@ -499,15 +499,15 @@ hipError_t launch_count_above(const double *e, long N, double eF, unsigned long 
 
 hipError_t launch_fo_flag(const double *eprev, const double *ecur, int nx, int ny, int nz, double eF,
                           long long *ids, long long cap, unsigned long long *count, unsigned long long *blk,
-                          hipStream_t st) {
+                          unsigned long long *masks, hipStream_t st) {
     const long M = (long)(nx - 1) * (ny - 1) * (nz > 1 ? nz - 1 : 1);
     if (M <= 0) return hipSuccess;
     const long nb = fo_flag_blocks(M);
     hipLaunchKernelGGL(fo_flag_count_kernel, dim3((unsigned)nb), dim3(256), 0, st, eprev, ecur, nx, ny, nz, eF, M,
-                       blk);
+                       blk, masks);
     hipLaunchKernelGGL(fo_flag_scan_kernel, dim3(1), dim3(1024), 0, st, blk, nb, count);
-    hipLaunchKernelGGL(fo_flag_write_kernel, dim3((unsigned)nb), dim3(256), 0, st, (const unsigned long long *)blk, ids,
-                       cap);
+    hipLaunchKernelGGL(fo_flag_write_kernel, dim3((unsigned)nb), dim3(256), 0, st, (const unsigned long long *)blk,
+                       (const unsigned long long *)masks, M, ids, cap);
     return hipGetLastError();
 }
 

@@ -56,13 +56,31 @@ hipError_t launch_admit_fp64(const AdmitSrc &S, double *q, double *e0, double *p
                              long N, long off, int nc, int *strikes, int *stop, hipStream_t st);
 hipError_t launch_count_above(const double *e, long N, double eF, unsigned long long *out, hipStream_t st);
 // The cut cubes' ids in increasing order into ids (capacity cap), their
-// number into *count; blk is scratch of fo_flag_scratch(cubes) entries: the
-// count, then the offset, of each block of 256 cubes, and its four waves' masks.
+// number into *count; blk is scratch of fo_flag_blocks(cubes) entries, the
+// count, then the offset, of each block of 256 cubes, and masks of
+// fo_flag_masks(cubes), the flags of each block's four waves.  Scratch of
+// fo_flag_scratch(cubes) entries holds both, the masks after the counts.
 inline constexpr long fo_flag_blocks(long cubes) { return (cubes + 255) / 256; }
-inline constexpr long fo_flag_scratch(long cubes) { return 5 * fo_flag_blocks(cubes); }
+inline constexpr long fo_flag_masks(long cubes) { return 4 * fo_flag_blocks(cubes); }
+inline constexpr long fo_flag_scratch(long cubes) { return fo_flag_blocks(cubes) + fo_flag_masks(cubes); }
+// The writing pass's place for the id of lane of wave w of a block of cubes
+// first to first + 255, or -1 where it has none: off is the block's offset, m0
+// to m3 its masks.  Scratch shared by calls that overlap can hold another
+// call's numbers; whatever they are, a place is in [0, cap) and its cube below M.
+__host__ __device__ __forceinline__ long long fo_flag_place(unsigned long long off, unsigned long long m0,
+                                                            unsigned long long m1, unsigned long long m2,
+                                                            unsigned long long m3, int w, int lane, long first, long M,
+                                                            long long cap) {
+    const unsigned long long mask = w < 2 ? (w ? m1 : m0) : (w == 2 ? m2 : m3);
+    unsigned long long pos = off + (unsigned long long)__builtin_popcountll(mask & ((1ull << lane) - 1ull));
+    pos += (unsigned long long)((w > 0 ? __builtin_popcountll(m0) : 0) + (w > 1 ? __builtin_popcountll(m1) : 0) +
+                                (w > 2 ? __builtin_popcountll(m2) : 0));
+    const bool flagged = (mask >> lane & 1) != 0;
+    return (int)flagged & (int)(first + 64 * w + lane < M) & (int)(pos < (unsigned long long)cap) ? (long long)pos : -1;
+}
 hipError_t launch_fo_flag(const double *eprev, const double *ecur, int nx, int ny, int nz, double eF,
                           long long *ids, long long cap, unsigned long long *count, unsigned long long *blk,
-                          hipStream_t st);
+                          unsigned long long *masks, hipStream_t st);
 hipError_t launch_fo_corners(const double *eprev, const double *ecur, int nx, int ny, int nz, const long long *ids,
                              long long n, double *corners, hipStream_t st);
 // The ten variables the freezeout surface interpolates (u^x u^y u^eta e pi^xx

@@ -14,6 +14,9 @@
 
 namespace {
 
+// The masks lie after the counts of the largest lattice, whatever the call's:
+// calls that overlap read each other's counts as counts and masks as masks.
+constexpr long MASKS_AT = vh::fo_flag_blocks(VH_FO_NOALLOC_MAX_CUBES);
 constexpr long MAX_SCRATCH = vh::fo_flag_scratch(VH_FO_NOALLOC_MAX_CUBES);
 constexpr int MAX_DEVICES = 64;
 
@@ -59,7 +62,7 @@ extern "C" vh_status vh_fo_flag_noalloc(const double *eprev, const double *ecur,
     // every block writes its own count and the scan writes the total, so
     // nothing is cleared first
     r = vh::launch_fo_flag(eprev, ecur, nx, ny, nz, eF, reinterpret_cast<long long *>(ids), (long long)cap,
-                           reinterpret_cast<unsigned long long *>(n_flagged), blk,
+                           reinterpret_cast<unsigned long long *>(n_flagged), blk, blk + MASKS_AT,
                            static_cast<hipStream_t>(stream));
     if (r != hipSuccess) {
         vh::set_last_error(std::string("vh_fo_flag_noalloc: ") + hipGetErrorString(r));

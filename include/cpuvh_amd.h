@@ -204,11 +204,13 @@ vh_status vh_fo_surface(vh_handle *h, const double *widths, int *n_el, double *e
  * device int64) receives the full count.  Enqueued on `stream` (a
  * hipStream_t, NULL for the null stream) of the current device, with no
  * synchronisation, so the call can be captured into a graph; the results are
- * there once the stream reaches them.  The kernels' per-block counts live in
- * one fixed device array of the library per GPU (2.5 MiB, kept until the
- * process ends): at most VH_FO_NOALLOC_MAX_CUBES cubes ((nx-1)(ny-1)(nz-1),
- * nz-1 read as 1 in 2+1D), else VH_ERR_ARG; calls that overlap on one GPU race
- * for that array. */
+ * there once the stream reaches them.  The kernels' per-block counts and flag
+ * masks live in one fixed device array of the library per GPU (2.5 MiB, kept
+ * until the process ends): at most VH_FO_NOALLOC_MAX_CUBES cubes
+ * ((nx-1)(ny-1)(nz-1), nz-1 read as 1 in 2+1D), else VH_ERR_ARG; calls that
+ * overlap on one GPU race for that array and may return a wrong count and
+ * wrong ids, other calls' cubes among them, though never more than cap ids and
+ * never one outside the lattice. */
 #define VH_FO_NOALLOC_MAX_CUBES 16777216L
 vh_status vh_fo_flag_noalloc(const double *eprev, const double *ecur, int nx, int ny, int nz, double eF,
                              int64_t *ids, int64_t cap, int64_t *n_flagged, void *stream);
