@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -114,6 +115,7 @@ struct vh_batch {
     int hslot_next = 0;
     float *qf[3][15] = {}, *qfl[3][4] = {}, *uf[3][4] = {}, *ef[2] = {}, *pf[2] = {};
     int tile2 = 0, tile3 = 0;
+    bool tile3_set = false;  // by the caller or the autotuner; else by mixed_tile_3d, per layout
     int face_mode = 1;  // the reference's face semantics (vh_batch_set_face_mode)
     bool layout_dirty = true;
     int layout_version = 0;
@@ -178,6 +180,12 @@ long event_blocks(const vh_batch *b, const Event &E) {
 
 vh_status rebuild_layout(vh_batch *b) {
     if (!b->layout_dirty) return VH_OK;
+    if (b->mixed && !b->tile3_set) {
+        std::vector<std::array<int, 3>> sizes;
+        for (const Event &E : b->ev)
+            if (E.used && E.prm.nz > 1) sizes.push_back({E.prm.nx, E.prm.ny, E.prm.nz});
+        if (!sizes.empty()) b->tile3 = mixed_tile_3d(sizes);
+    }
     std::vector<int> bev, bfirst, cev;
     std::vector<long> cstart;
     int n2 = 0, n2bi = 0;
@@ -1174,6 +1182,8 @@ vh_status vh_batch_autotune(vh_batch *b, int reps, int *tile2d, int *tile3d) {
     // admitted the first two are within a few per cent of each other.
     constexpr float MARGIN = 0.02f;
     const int start[2] = {b->tile2, b->tile3};
+    const bool was_set = b->tile3_set;
+    b->tile3_set = true;
     int best[2] = {b->tile2, b->tile3};
     for (int dim = 0; dim < 2; ++dim) {
         std::vector<float> t[MIXED_NTILE];
@@ -1207,6 +1217,7 @@ vh_status vh_batch_autotune(vh_batch *b, int reps, int *tile2d, int *tile3d) {
             }
         if (!any) {
             best[dim] = start[dim];
+            if (dim == 1) b->tile3_set = was_set;
         } else {
             float med[MIXED_NTILE];
             for (int v = 0; v < MIXED_NTILE; ++v) {
@@ -1233,6 +1244,7 @@ vh_status vh_batch_set_tiles(vh_batch *b, int tile2d, int tile3d) {
     if (!b->mixed) return VH_OK;
     b->tile2 = tile2d;
     b->tile3 = tile3d;
+    b->tile3_set = true;
     b->layout_dirty = true;
     return VH_OK;
 }

@@ -2,7 +2,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <string>
+#include <vector>
+
 #include "vh_stage.hpp"
 #include "vh_host_eos.hpp"
 
@@ -169,8 +172,43 @@ namespace mx {
 struct MxFields;
 }
 constexpr int MIXED_NTILE = 3;
-extern const int MIXED_TILES_2D[MIXED_NTILE][3];  // (TX, TY, TZ) of each 2+1D tile variant
-extern const int MIXED_TILES_3D[MIXED_NTILE][3];
+// (TX, TY, TZ) of each tile variant
+inline constexpr int MIXED_TILES_2D[MIXED_NTILE][3] = {{16, 15, 1}, {32, 7, 1}, {64, 3, 1}};
+inline constexpr int MIXED_TILES_3D[MIXED_NTILE][3] = {{16, 4, 3}, {6, 6, 6}, {8, 4, 6}};
+// The 3+1D variant of a launch over events of the given (nx, ny, nz), where
+// none was set: the least cost of its cells, rows counted in whole tiles.
+// Rows decide, since a load touches as many cache lines as its lanes touch
+// rows: a cell in rows of 6 costs 1.45 times one in rows of 16 (201x201x101,
+// 1,600 against 1,103 us a launch), one in rows of 8 1.09 times; it is weighed
+// 1.21 because between 33 and 56 cells a row the two measure within 10 % of each
+// other either way, and rows of 16 are then the better with many cells.  ny
+// counts in whole tiles only where it is at most 5 (16x4x3 and 8x4x6 then work on
+// 8 rows, 6x6x6 on 6); counting it everywhere takes 6x6x6 where 16x4x3 is up to
+// 1.5 times as fast.  Over 1,189 batches of 1 to 16 equal events (nx 3 to 131,
+// nine shapes of ny x nz, table and conformal) this choice takes 0.84 of 6x6x6's
+// time in the geometric mean and 3 % more than the best of the three; it is more
+// than 18 % slower than 6x6x6 only in slabs of two or three cells along eta with
+// one or two cells in a row's last tile (50x33x3: 49 against 35 us a stage).
+// 16x4x3 alone takes up to 2.3 times 6x6x6's (16 events of 5x65x33: 155 against
+// 80 us, 64 of 17x17x17: 211 against 152).
+inline int mixed_tile_3d(const std::vector<std::array<int, 3>> &sizes) {
+    constexpr double COST[MIXED_NTILE] = {1.0, 1.45, 1.21};
+    int pick = 0;
+    double least = 0.0;
+    for (int v = 0; v < MIXED_NTILE; ++v) {
+        const int TX = MIXED_TILES_3D[v][0], TY = MIXED_TILES_3D[v][1];
+        double c = 0.0;
+        for (const auto &[nx, ny, nz] : sizes) {
+            const int x = (nx + TX - 1) / TX * TX, y = ny <= 5 ? (ny + TY - 1) / TY * TY : ny;
+            c += COST[v] * x * y * nz;
+        }
+        if (v == 0 || c < least) {
+            pick = v;
+            least = c;
+        }
+    }
+    return pick;
+}
 // bi: the launch holds only boost-invariant 2+1D events (nz = 1, u^eta and
 // the pi^{. eta} components zero), whose eta components stay zero.
 hipError_t launch_stage_mixed(const mx::MxFields &F, const EosDev &E, int nc, bool dim3d, int tile, bool bi,

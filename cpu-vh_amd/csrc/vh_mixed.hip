@@ -81,7 +81,8 @@ hipError_t launch_mx(const mx::MxFields &F, const EosDev &E, const EvDesc *ev, c
 // with admission and downloads: 6x6x6 150.9 ms, 8x8x3 125.7, 8x4x6 120.8,
 // 16x4x3 110.9, 16x3x4 109.0; four events of 60 to 111 cells a side, 41 deep,
 // 47.4, 37.4, 35.9, 33.7, 34.2 ms.  12x4x4 (116.5), 21x3x3 (121.6) and 10x5x4
-// lie between.  In 2+1D 21x11, 18x13 and 25x9 measured 5 % slower than 16x15.
+// lie between.  6x6x6 and 8x4x6 are there for lattices whose rows would leave
+// most of a 16-cell row empty (mixed_tile_3d).  In 2+1D 21x11, 18x13 and 25x9 measured 5 % slower than 16x15.
 // bi: every event of the launch is a boost-invariant 2+1D event (the
 // kernels that neither load nor evolve the eta components).
 template <int NC, bool TABLE>
@@ -102,7 +103,7 @@ hipError_t launch_mx_tile(const mx::MxFields &F, const EosDev &E, bool dim3d, in
     } else {
         switch (tile) {
         case 0: return launch_mx<NC, TABLE, true, 16, 4, 3>(F, E, ev, blk_ev, blk_first, nblocks, st);
-        case 1: return launch_mx<NC, TABLE, true, 16, 3, 4>(F, E, ev, blk_ev, blk_first, nblocks, st);
+        case 1: return launch_mx<NC, TABLE, true, 6, 6, 6>(F, E, ev, blk_ev, blk_first, nblocks, st);
         case 2: return launch_mx<NC, TABLE, true, 8, 4, 6>(F, E, ev, blk_ev, blk_first, nblocks, st);
         }
     }
@@ -110,9 +111,6 @@ hipError_t launch_mx_tile(const mx::MxFields &F, const EosDev &E, bool dim3d, in
 }
 
 }  // namespace
-
-const int MIXED_TILES_2D[MIXED_NTILE][3] = {{16, 15, 1}, {32, 7, 1}, {64, 3, 1}};
-const int MIXED_TILES_3D[MIXED_NTILE][3] = {{16, 4, 3}, {16, 3, 4}, {8, 4, 6}};
 
 hipError_t launch_stage_mixed(const mx::MxFields &F, const EosDev &E, int nc, bool dim3d, int tile, bool bi,
                               const EvDesc *ev, const int *blk_ev, const int *blk_first, int nblocks, hipStream_t st) {

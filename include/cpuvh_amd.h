@@ -468,7 +468,9 @@ vh_status vh_batch_free_cells(vh_batch *b, int64_t *free_cells, int64_t *largest
  * on the resident events (the state is not advanced) and keeps the 2+1D and
  * 3+1D tiles by median time, a later variant replacing the one kept only
  * when more than 2 % faster (variant 0 is the fastest over whole runs of 2+1D
- * Glauber batches).  FP64 batches: no variants, *tile = -1. */
+ * Glauber batches).  FP64 batches: no variants, *tile = -1.  Where neither call
+ * was made the 2+1D tile is variant 0 and the 3+1D tile the one the resident
+ * events' rows fit; every variant gives the same bits. */
 vh_status vh_batch_autotune(vh_batch *b, int reps, int *tile2d, int *tile3d);
 vh_status vh_batch_set_tiles(vh_batch *b, int tile2d, int tile3d);
 /* Mixed form: how face fluxes are shared.  The reference evaluates each face
