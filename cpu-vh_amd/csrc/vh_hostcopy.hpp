@@ -10,6 +10,7 @@
 // field crosses as it is stored and is widened on the way out.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <xmmintrin.h>
 
 #include <algorithm>
 #include <cstring>
@@ -70,13 +71,21 @@ class HostCopy {
                 return r;
             },
             [&](const double *b, size_t at, size_t len) {
-                const float *h = reinterpret_cast<const float *>(b), *l = h + len;
-                double *o = out + at;
-                if (lo)
-                    for (size_t i = 0; i < len; ++i) o[i] = (double)h[i] + (double)l[i];
-                else
-                    for (size_t i = 0; i < len; ++i) o[i] = (double)h[i];
+                const float *h = reinterpret_cast<const float *>(b);
+                widen(out + at, h, lo ? h + len : nullptr, len);
             });
+    }
+    // out = hi (+ lo where not null), whatever the calling thread's MXCSR says:
+    // a thread that takes subnormals as zero (torch.set_flush_denormal, programs
+    // built with -ffast-math) gets an FP32 field's subnormal values all the same.
+    __attribute__((noinline)) static void widen(double *out, const float *hi, const float *lo, size_t n) {
+        const unsigned mxcsr = _mm_getcsr();
+        _mm_setcsr(mxcsr & ~0x8040u);  // neither denormals-are-zero nor flush-to-zero
+        if (lo)
+            for (size_t i = 0; i < n; ++i) out[i] = (double)hi[i] + (double)lo[i];
+        else
+            for (size_t i = 0; i < n; ++i) out[i] = (double)hi[i];
+        _mm_setcsr(mxcsr);
     }
 
   private:
