@@ -184,9 +184,9 @@ vh_status enqueue_step(vh_handle *h, const StepTimes &st, const StepTimes *tab, 
 }
 
 vh_status check_err(vh_handle *h) {
-    HIPCHK(h->host.fetch_err(h->d_err, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    return h->host.err()[0] ? VH_ERR_NAN : VH_OK;
+    bool err = false;
+    HIPCHK(h->host.status(h->d_err, h->stream, &err));
+    return err ? VH_ERR_NAN : VH_OK;
 }
 
 }  // namespace
@@ -523,8 +523,9 @@ vh_status vh_download(vh_handle *h, int field, double *out) {
         HIPCHK(hipMemcpyAsync(out, src, sizeof(double) * h->N, hipMemcpyDeviceToHost, h->stream));
         return check_err(h);
     }
-    HIPCHK(h->host.fetch(out, src, h->N, h->d_err, h->stream));
-    return h->host.err()[0] ? VH_ERR_NAN : VH_OK;
+    bool err = false;
+    HIPCHK(h->host.fetch(out, src, h->N, h->d_err, h->stream, &err));
+    return err ? VH_ERR_NAN : VH_OK;
 }
 
 vh_status vh_thermal_vorticity(vh_handle *h) {

@@ -811,23 +811,23 @@ vh_status vh_batch_run(vh_batch *b, double eF, int coarse, int nchecks, int32_t 
     return st;
 }
 
-// The status of work that has ended, the error words copied to b->host.
-static vh_status ended(vh_batch *b) {
+// The status of work that has ended, err whether its error word is set.
+static vh_status ended(vh_batch *b, bool err) {
     if (b->timed) {
         float ms = 0;
         BCHK(hipEventElapsedTime(&ms, b->ev0, b->ev1));
         b->last_ms = ms;
         b->timed = false;
     }
-    return b->host.err()[0] ? VH_ERR_NAN : VH_OK;
+    return err ? VH_ERR_NAN : VH_OK;
 }
 
 vh_status vh_batch_sync(vh_batch *b) {
     if (!b) return VH_ERR_ARG;
     BCHK(hipSetDevice(b->dev));
-    BCHK(b->host.fetch_err(b->d_err, b->stream));
-    BCHK(hipStreamSynchronize(b->stream));
-    return ended(b);
+    bool err = false;
+    BCHK(b->host.status(b->d_err, b->stream, &err));
+    return ended(b, err);
 }
 
 double vh_batch_last_ms(const vh_batch *b) { return b ? b->last_ms : 0.0; }
@@ -864,8 +864,9 @@ vh_status vh_batch_download(vh_batch *b, int id, int field, double *out) {
             BCHK(hipMemcpyAsync(out, src + E.off, sizeof(double) * E.N, hipMemcpyDeviceToHost, b->stream));
             return vh_batch_sync(b);
         }
-        BCHK(b->host.fetch(out, src + E.off, E.N, b->d_err, b->stream));
-        return ended(b);
+        bool err = false;
+        BCHK(b->host.fetch(out, src + E.off, E.N, b->d_err, b->stream, &err));
+        return ended(b, err);
     }
     const float *hi = nullptr, *lo = nullptr;
     if (!field_of_mixed(b, field, flip, &hi, &lo)) return VH_ERR_ARG;
@@ -875,8 +876,9 @@ vh_status vh_batch_download(vh_batch *b, int id, int field, double *out) {
         return vh_batch_sync(b);
     }
     if (!HostCopy::registered(out)) {
-        BCHK(b->host.fetch_widened(out, hi + E.off, lo ? lo + E.off : nullptr, E.N, b->d_err, b->stream));
-        return ended(b);
+        bool err = false;
+        BCHK(b->host.fetch_widened(out, hi + E.off, lo ? lo + E.off : nullptr, E.N, b->d_err, b->stream, &err));
+        return ended(b, err);
     }
     double *tmp = nullptr;
     BCHK(hipMalloc(&tmp, sizeof(double) * E.N));

@@ -45,24 +45,29 @@ class HostCopy {
         }
         return a.type != hipMemoryTypeUnregistered;
     }
-    // Pinned copy of the three error words, valid after the wait.
-    int *err() { return reinterpret_cast<int *>(buf_ + 2 * half_); }
-    hipError_t fetch_err(const int *d_err, hipStream_t st) {
-        return hipMemcpyAsync(err(), d_err, 3 * sizeof(int), hipMemcpyDeviceToHost, st);
+    // Whether the error word is set once the stream's work has ended; waits.
+    hipError_t status(const int *d_err, hipStream_t st, bool *err) {
+        std::lock_guard<std::mutex> lock(mu_);
+        hipError_t r = fetch_err(d_err, st);
+        const hipError_t w = hipStreamSynchronize(st);
+        if (r == hipSuccess) r = w;
+        if (r == hipSuccess) *err = words()[0] != 0;
+        return r;
     }
-    // n doubles and the error words; waits.
-    hipError_t fetch(double *out, const double *src, size_t n, const int *d_err, hipStream_t st) {
+    // n doubles, and whether the error word is set; waits.
+    hipError_t fetch(double *out, const double *src, size_t n, const int *d_err, hipStream_t st, bool *err) {
         return chunks(
-            n, d_err, st,
+            n, d_err, st, err,
             [&](double *b, size_t at, size_t len) {
                 return hipMemcpyAsync(b, src + at, len * sizeof(double), hipMemcpyDeviceToHost, st);
             },
             [&](const double *b, size_t at, size_t len) { std::memcpy(out + at, b, len * sizeof(double)); });
     }
-    // n values hi (+ lo where not null), widened; waits.
-    hipError_t fetch_widened(double *out, const float *hi, const float *lo, size_t n, const int *d_err, hipStream_t st) {
+    // n values hi (+ lo where not null), widened, and whether the error word is set; waits.
+    hipError_t fetch_widened(double *out, const float *hi, const float *lo, size_t n, const int *d_err, hipStream_t st,
+                             bool *err) {
         return chunks(
-            n, d_err, st,
+            n, d_err, st, err,
             [&](double *b, size_t at, size_t len) {
                 float *f = reinterpret_cast<float *>(b);
                 hipError_t r = hipMemcpyAsync(f, hi + at, len * sizeof(float), hipMemcpyDeviceToHost, st);
@@ -91,9 +96,13 @@ class HostCopy {
   private:
     static constexpr size_t MAX_HALF = size_t(1) << 17;  // doubles: 1 MiB, within a core's L2
     static constexpr size_t ERR_BYTES = 64;
+    int *words() { return reinterpret_cast<int *>(buf_ + 2 * half_); }  // the three error words
+    hipError_t fetch_err(const int *d_err, hipStream_t st) {
+        return hipMemcpyAsync(words(), d_err, 3 * sizeof(int), hipMemcpyDeviceToHost, st);
+    }
     template <class COPY, class TAKE>
-    hipError_t chunks(size_t n, const int *d_err, hipStream_t st, COPY &&copy, TAKE &&take) {
-        std::lock_guard<std::mutex> lock(mu_);  // downloads of one owner from two threads take turns
+    hipError_t chunks(size_t n, const int *d_err, hipStream_t st, bool *err, COPY &&copy, TAKE &&take) {
+        std::lock_guard<std::mutex> lock(mu_);
         const size_t count = (n + half_ - 1) / half_;
         auto start = [&](size_t c) {
             hipError_t r = copy(buf_ + (c & 1) * half_, c * half_, std::min(half_, n - c * half_));
@@ -107,9 +116,10 @@ class HostCopy {
             if (r == hipSuccess) take(buf_ + (c & 1) * half_, c * half_, std::min(half_, n - c * half_));
         }
         if (r != hipSuccess) (void)hipStreamSynchronize(st);  // no copy still writes the buffer
+        else *err = words()[0] != 0;
         return r;
     }
-    std::mutex mu_;
+    std::mutex mu_;  // held from the first copy into the pinned memory to its last reading: threads take turns
     double *buf_ = nullptr;
     size_t half_ = 0;
     hipEvent_t full_[2] = {};
