@@ -222,14 +222,15 @@ __device__ __forceinline__ void dir_contrib(const StageParams &P, const GEO &G, 
         for (int q = 0; q < 4; ++q) sd[q] = Side{dir == 0 ? w[q].ux : (dir == 1 ? w[q].uy : w[q].un), div.recip(w[q].ut)};
     }
     const Side Rf = sd[0], Lf = sd[1], Rb = sd[2], Lb = sd[3];
-    const double af = face_speed(Rf, Lf, div), ab = face_speed(Rb, Lb, div);
+    const double af = checked(div, [&](auto &dv) { return face_speed(Rf, Lf, dv); });
+    const double ab = checked(div, [&](auto &dv) { return face_speed(Rb, Lb, dv); });
 
     // Per-variable fluxes of both faces, then r.  pi and Pi come first, so that
     // the pi-gradient terms of T^{tau mu} (central differences, fac = 1/d/2)
     // are formed from the same lines, without eighteen loads of their own (131x131x61,
     // 60 steps with copies: 97.8 -> 96.0 ms; 45x37x23: 4.87 -> 4.78 ms).
     const double fac = 1 / d / 2;
-    const double v = div(v_c, rut);
+    const double v = checked(div, [&](auto &dv) { return dv(v_c, rut); });
     double dT[4], dA[4] = {}, dPi = 0.0, S[4];
     Points next = load_line(P.q[4], sm2, sm1, s, sp1, sp2);
 #pragma unroll
@@ -259,11 +260,11 @@ __device__ __forceinline__ void dir_contrib(const StageParams &P, const GEO &G, 
             }
         }
         const Line l = make_line(now);
-        const double Hf = face_var_flux(Rf, Lf, af, right_fwd(l), left_fwd(l), div);
-        const double Hb = face_var_flux(Rb, Lb, ab, right_bwd(l), left_bwd(l), div);
-        double r = -Hf;
-        r += Hb;
-        r = div(r, rd);
+        double r = checked(div, [&](auto &dv) {
+            const double Hf = face_var_flux(Rf, Lf, af, right_fwd(l), left_fwd(l), dv);
+            const double Hb = face_var_flux(Rb, Lb, ab, right_bwd(l), left_bwd(l), dv);
+            return dv(-Hf + Hb, rd);
+        });
         if (n < 4) r += S[n];
         r *= G.dt;
         sink(n, r);
@@ -288,7 +289,7 @@ __device__ __forceinline__ void source_init(const StageParams &P, const GEO &G, 
                                             SINK &&sink, DV &div) {
     const Recip rdx = div.recip(G.dx), rdy = div.recip(G.dy), rdz = div.recip(G.dz);
     const Recip rt = div.recip(t), rdt = div.recip(G.dt), rt2pow = div.recip(t2pow), rut = div.recip(ut);
-    const Recip r3{3.0, 1.0 / 3.0, true}, r5{5.0, 1.0 / 5.0, true};
+    const IntRecip r3{3.0, 1.0 / 3.0}, r5{5.0, 1.0 / 5.0};
     auto put = [&](int n, double Sn) { sink(n, P.q[n][s] + G.dt * Sn); };
     const double ttt = P.q[0][s], ttx = P.q[1][s], tty = P.q[2][s], ttn = P.q[3][s];
     const double pitt = P.q[4][s], pitx = P.q[5][s], pity = P.q[6][s], pitn = P.q[7][s], pixx = P.q[8][s],

@@ -47,6 +47,23 @@ long part(const char *name, long n, int alo, int ahi, int blo, int bhi, bool all
     return wrong;
 }
 
+// quotients by 3 and 5: nothing refused
+long by_integers(const char *name, long n, int alo, int ahi) {
+    const vh::IntRecip r3{3.0, 1.0 / 3.0}, r5{5.0, 1.0 / 5.0};
+    long bad = 0, refused = 0;
+    for (long i = 0; i < n; ++i) {
+        const double a = i < 4096 ? (i & 1 ? -1 : 1) * (double)(i >> 1) * 0x1p-1074 : make(between(alo, ahi), false);
+        vh::DivTry d;
+        const double q3 = d(a, r3), q5 = d(a, r5);
+        d.see(q3);
+        d.see(q5);
+        refused += d.fails();
+        bad += !same(q3, a / 3.0) || !same(q5, a / 5.0);
+    }
+    std::printf("%s: mismatches %ld refused %ld of %ld%s\n", name, bad, refused, n, bad || refused ? " WRONG" : "");
+    return bad || refused;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -62,5 +79,7 @@ int main(int argc, char **argv) {
     wrong += part("quotients of the last bits", n, -1074, -1060, -4, 8, false);
     wrong += part("overflowing quotients", n, 1000, 1023, -16, 20, false);
     wrong += part("divisors outside", n, -960, 800, -140, 140, false);
+    wrong += by_integers("thirds and fifths", n, -1022, 1023);
+    wrong += by_integers("subnormal thirds and fifths", n, -1074, -1000);
     return wrong ? 1 : 0;
 }
