@@ -622,6 +622,36 @@ def run_dropin_3d(w, table, steps, warmup):
     }
 
 
+# What the one line holds of the record: who reads it keeps its last few
+# thousand characters.  The rest, the error reports above all, goes to --details.
+LINE_KEYS = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+             "vs_baseline", "dtype", "data", "config", "speedup_vs_plain_fp64", "speedup_vs_plain_fp64_incl_setup",
+             "speedup_vs_cpu_reference")
+LINE_PARTS = {
+    "accuracy": ("pass_metric_bar", "pass_attainable_bar", "pass_attainable_bar_q999"),
+    "batched_mixed": ("events_per_s", "events_per_s_excl_admission", "events_failed", "zone_upd_per_s"),
+    "batched_fp64": ("events_per_s", "events_failed", "zone_upd_per_s"),
+    "plain_fp64_loop": ("events_per_s", "events_per_s_excl_setup", "zone_upd_per_s"),
+    "fp64_dropin_3d": ("cells", "steps", "ms_per_step", "zone_upd_per_s", "events_per_s_at_600_steps"),
+    "precision_form_3d": ("steps", "cells", "fp64_s", "mixed_s"),
+    "roofline": ("bound", "achieved", "peak", "unit", "frac", "traffic", "kernel", "avg_launch_ms",
+                 "algorithmic_bytes_per_zone_update"),
+    "cpu_baseline": ("value", "unit", "cores", "kind", "events_per_s"),
+}
+SERVING_KEYS = ("rate_per_s", "requests", "completed", "events_per_s", "zone_upd_per_s", "p50_s", "p99_s")
+
+
+def headline(out):
+    """The record's one line."""
+    line = {k: out[k] for k in LINE_KEYS if k in out}
+    for part, keys in LINE_PARTS.items():
+        if out.get(part):
+            line[part] = {k: out[part][k] for k in keys if k in out[part]}
+    if out.get("serving"):
+        line["serving"] = [{k: r[k] for k in SERVING_KEYS if k in r} for r in out["serving"]["sweep"]]
+    return line
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -656,6 +686,7 @@ def main():
     ap.add_argument("--reference-bulk", action="store_true",
                     help="the reference's c_s^2 (1/3 on this table: bulk terms zero) instead of the table's sound "
                          "speed with zeta/s(T) peaked at 160 MeV")
+    ap.add_argument("--details", default=None, help="file for the whole record: every leg, checkpoint and error quantile")
     ap.add_argument("--copy-probe", action="store_true",
                     help="only copy 512 MiB device to device (scale of the HBM byte counters)")
     args = ap.parse_args()
@@ -826,7 +857,10 @@ def main():
     }
     if cpu and "events_per_s" in cpu and gpu_const:
         out["speedup_vs_cpu_reference"] = gpu_const["events_per_s_excl_admission"] / cpu["events_per_s"]
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(headline(out)))
     return 0
 
 
