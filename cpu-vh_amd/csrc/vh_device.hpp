@@ -174,8 +174,9 @@ __device__ __forceinline__ float sqrt_mid(float x) {
 // or infinite, which see() notes.  DivFast compares, selects and branches
 // at each of about 300 divisions a cell and stage (three 64-bit compares, a
 // select and a branch each); here a division costs its four instructions and
-// two 32-bit ones.  With nr_step_try the 3+1D kernel issues 2.36e8 VALU
-// instructions per launch at 131x131x61 where it issued 3.35e8; with their
+// two 32-bit ones.  With nr_step_try the 3+1D kernel issued 2.36e8 VALU
+// instructions per launch at 131x131x61 (2.23e8 with checked() and IntRecip
+// since) where it issued 3.35e8; with their
 // copies, 60 steps of that event took 112.8 instead of 122.8 ms, 100 steps of
 // a 147x129 event 6.48 instead of 8.32 ms, 200 conformal steps at 201x201 9.87
 // instead of 12.2 ms, 40 steps of 16 batched events 16.6 instead of 18.9 ms.

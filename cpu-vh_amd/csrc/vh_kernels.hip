@@ -127,8 +127,9 @@ __device__ __forceinline__ bool fo_cut(const double *__restrict__ eprev, const d
 // the cut cubes of each block of 256 and keeps its waves' masks, pass 2 turns
 // the counts into offsets, pass 3 writes each id at its block's offset plus
 // its rank in the block.  The masks (a bit a cube) stand in for a second
-// evaluation of the flags, sixteen loads a cube: 27.2 -> 20.3 us a call at
-// 131x131x61 among others, of which some 12 are the three launches.
+// evaluation of the flags, sixteen loads a cube: 27.2 -> 20.1 us a call at
+// 131x131x61 among others, of which some 12 are the three launches; below some
+// 1e5 cubes the launches are all of it, 11 us either way.
 __global__ __launch_bounds__(256) void fo_flag_count_kernel(const double *__restrict__ eprev,
                                                             const double *__restrict__ ecur, int nx, int ny, int nz,
                                                             double eF, long M, unsigned long long *__restrict__ blk,
